@@ -11,6 +11,7 @@ __device__ uint32_t xpu_stamp_phase[xpu::kPhaseSlots * xpu::kStampRing * xpu::kP
 #include "gemv.hip"
 #include "synth.hip"
 #include "qwen3_ops.hip"
+#include "prefill_gemv.hip"
 #include "gemm.hip"
 #include "prefill_attention.hip"
 #include "peak.hip"

@@ -180,6 +180,12 @@ struct xpu_qwen3 {
                         *pf_qkv_k = nullptr, *pf_o_k = nullptr, *pf_gu_k = nullptr, *pf_down_k = nullptr;
   // rows per wavefront of those four batched GEMV kernels (their _r<R>)
   uint32_t pf_qkv_r = 0, pf_o_r = 0, pf_gu_r = 0, pf_down_r = 0;
+  // the same projections on the FP32 MFMA (kernels/prefill_gemv.hip), for
+  // chunks of more than kRowsFrom tokens, and their block sizes
+  struct Rows {
+    const xpu::KernelInfo *k = nullptr;
+    uint32_t block = 0;
+  } pf_qkv_m, pf_o_m, pf_gu_m, pf_down_m;
 
   ~xpu_qwen3() {
     if (graph) xpu_rt_graph_destroy(graph);
@@ -440,6 +446,22 @@ int setup_prefill(xpu_qwen3 &e) {
   e.pf_o_k = gemv(1, qd, e.pf_o_r);
   e.pf_gu_k = gemv(2, c.hidden, e.pf_gu_r);
   e.pf_down_k = gemv(1, c.intermediate, e.pf_down_r);
+  auto rows = [&](int epi, uint32_t K) {
+    xpu_qwen3::Rows r;
+    for (uint32_t waves : {4u, 8u}) {
+      r.k = e.rt->find_exact("xpu_q3_pf_rows_e" + std::to_string(epi) + "_c" + std::to_string(K / 512u) + "_w" +
+                             std::to_string(waves));
+      r.block = 64u * waves;
+      if (r.k) break;
+    }
+    return r;
+  };
+  if (e.pf_qkv_k && e.pf_o_k && e.pf_gu_k && e.pf_down_k) {
+    e.pf_qkv_m = rows(0, c.hidden);
+    e.pf_o_m = rows(1, qd);
+    e.pf_gu_m = rows(2, c.hidden);
+    e.pf_down_m = rows(1, c.intermediate);
+  }
   e.pf_embed_k = e.rt->find_exact("xpu_q3_pf_embed");
   e.pf_norm_k = e.rt->find_exact("xpu_q3_pf_rmsnorm");
   e.pf_rope_k = e.rt->find_exact("xpu_q3_pf_rope_cache");
@@ -471,6 +493,32 @@ int setup_prefill(xpu_qwen3 &e) {
   e.batched_prefill = e.pf_ok;  // the default: the bit-identical form; the GEMM form is opt-in
   return e.pf_ok ? size_prompt_buffers(e, false) : XPU_OK;
 }
+
+// Token groups of a batched projection on the FP32 MFMA: blocks of 16 rows
+// and ceil(tiles / groups) token tiles, spread evenly over the compute units,
+// cost the busiest unit ceil(row tiles * groups / CUs) blocks of that many
+// tiles; the least such cost, and among equals the first that gives every
+// unit two blocks (their loads hide each other's latency), else the most
+// groups. Measured at 128 and 256 tokens: within 3% of the best group count
+// for all four 0.6B projections (a count off the rule costs up to 40%).
+uint32_t rows_groups(uint32_t compute_units, uint32_t row_tiles, uint32_t token_tiles) {
+  uint32_t best = 1;
+  uint64_t best_cost = ~uint64_t{0};
+  for (uint32_t g = 1; g <= token_tiles; ++g) {
+    const uint64_t cost = (uint64_t{row_tiles} * g + compute_units - 1) / compute_units *
+                          ((token_tiles + g - 1) / g);
+    if (cost < best_cost || (cost == best_cost && uint64_t{row_tiles} * best < 2ull * compute_units)) {
+      best = g;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+// Chunks of more tokens take the FP32 MFMA kernels, whose token tiles are 16
+// wide: at 25-32 tokens the four 0.6B projections take 44.0 us against 46.4
+// on the VALU kernels, at 17-24 tokens 43.0 against 39.7, at 48 51 against 62.
+constexpr uint32_t kRowsFrom = 24;
 
 int launch(xpu_qwen3 &e, const xpu_qwen3::Launch &l, uint32_t block, std::initializer_list<xpu_kernel_arg> args) {
   return e.rt->launch(*l.k, l.grid, 1, block, l.shared, args.begin(), static_cast<uint32_t>(args.size()));
@@ -589,6 +637,13 @@ int run_prefill(xpu_qwen3 &e, uint32_t P, bool head) {
     // launch that fills the blocks per compute unit its registers and LDS
     // allow (measured: QKV and [gate; up] 3/2, o_proj 2, down_proj 2)
     auto groups = [&](uint32_t r, uint32_t base) { return T > 8 ? std::max(1u, r / base) : 1u; };
+    // a projection on the FP32 MFMA: M output rows of 16-row tiles
+    auto on_rows = [&](const xpu_qwen3::Rows &r, const uint16_t *w, const uint16_t *in, uint16_t *out, uint32_t M) {
+      uint32_t g = rows_groups(rt->compute_units, M / 16, (T + 15) / 16);
+      return go(r.k, (M / 16 + 7) / 8 * 8 * g, 1, r.block, 0,
+                {{8, &w}, {8, &in}, {8, &out}, {4, &M}, {4, &T}, {4, &g}});
+    };
+    const bool rows = T > kRowsFrom && e.pf_qkv_m.k && e.pf_o_m.k && e.pf_gu_m.k && e.pf_down_m.k;
     if ((rc = go(e.pf_embed_k, T, 1, 256, 0, {{8, &e.embed}, {8, &e.prompt}, {4, &p0}, {8, &e.pf_x}, {4, &H}, {4, &V}})))
       return rc;
     // the GEMM form's split-K reductions of o_proj and down_proj can write
@@ -604,6 +659,8 @@ int run_prefill(xpu_qwen3 &e, uint32_t P, bool head) {
       xn_ready = false;
       if (e.gemm_prefill) {
         if ((rc = xpu::gemm_nt(rt, e.pf_xn, L.qkv, e.pf_qkv, T, qkv_rows, H, false))) return rc;
+      } else if (rows) {
+        if ((rc = on_rows(e.pf_qkv_m, L.qkv, e.pf_xn, e.pf_qkv, qkv_rows))) return rc;
       } else if ((rc = go(e.pf_qkv_k, (qkv_rows + 4 * e.pf_qkv_r - 1) / (4 * e.pf_qkv_r), groups(e.pf_qkv_r, 2) * (T > 8 ? 3u : 2u) / 2u, 256,
                           pf_lds(H),
                           {{8, &L.qkv}, {8, &e.pf_xn}, {8, &e.pf_qkv}, {4, &qkv_rows}, {4, &T}}))) {
@@ -641,6 +698,8 @@ int run_prefill(xpu_qwen3 &e, uint32_t P, bool head) {
       if (e.gemm_prefill) {
         if ((rc = xpu::gemm_nt(rt, e.pf_a, L.o, e.pf_x, T, H, qd, true, L.post_norm, e.pf_xn, eps, &normed)))
           return rc;
+      } else if (rows) {
+        if ((rc = on_rows(e.pf_o_m, L.o, e.pf_a, e.pf_x, H))) return rc;
       } else if ((rc = go(e.pf_o_k, (H + 4 * e.pf_o_r - 1) / (4 * e.pf_o_r), groups(e.pf_o_r, 1) * (T > 8 ? 2u : 1u), 256, pf_lds(qd),
                           {{8, &L.o}, {8, &e.pf_a}, {8, &e.pf_x}, {4, &H}, {4, &T}}))) {
         return rc;
@@ -659,6 +718,11 @@ int run_prefill(xpu_qwen3 &e, uint32_t P, bool head) {
         if ((rc = xpu::gemm_nt(rt, e.pf_h, L.down, e.pf_x, T, H, I, true, e.layers[l + 1].in_norm, e.pf_xn, eps,
                                &xn_ready)))
           return rc;
+        continue;
+      }
+      if (rows) {
+        if ((rc = on_rows(e.pf_gu_m, L.gu, e.pf_xn, e.pf_h, I))) return rc;
+        if ((rc = on_rows(e.pf_down_m, L.down, e.pf_h, e.pf_x, H))) return rc;
         continue;
       }
       if ((rc = go(e.pf_gu_k, (I + 2 * e.pf_gu_r - 1) / (2 * e.pf_gu_r), groups(e.pf_gu_r, 2) * (T > 8 ? 3u : 2u) / 2u,
