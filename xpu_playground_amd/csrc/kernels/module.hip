@@ -12,6 +12,7 @@ __device__ uint32_t xpu_stamp_phase[xpu::kPhaseSlots * xpu::kStampRing * xpu::kP
 #include "synth.hip"
 #include "qwen3_ops.hip"
 #include "prefill_gemv.hip"
+#include "prefill_attention_rows.hip"
 #include "gemm.hip"
 #include "prefill_attention.hip"
 #include "peak.hip"

@@ -175,6 +175,7 @@ struct xpu_qwen3 {
   uint16_t *pf_x = nullptr, *pf_xn = nullptr, *pf_qkv = nullptr, *pf_q = nullptr, *pf_a = nullptr,
            *pf_h = nullptr, *pf_gu = nullptr;
   const xpu::KernelInfo *pf_silu_k = nullptr, *pf_attn_mfma_k = nullptr;
+  const xpu::KernelInfo *pf_attn_rows_k = nullptr;  // 16 queries per block on the FP32 MFMA, contexts up to 4096
   const xpu::KernelInfo *pf_attn_short_k = nullptr;  // chunks whose contexts stay within 256 positions
   const xpu::KernelInfo *pf_embed_k = nullptr, *pf_norm_k = nullptr, *pf_rope_k = nullptr, *pf_attn_k = nullptr,
                         *pf_qkv_k = nullptr, *pf_o_k = nullptr, *pf_gu_k = nullptr, *pf_down_k = nullptr;
@@ -426,6 +427,11 @@ int size_prompt_buffers(xpu_qwen3 &e, bool gemm) {
   return XPU_OK;
 }
 
+constexpr uint32_t kBatchedChunk = 1024;
+// LDS of xpu_q3_pf_attention_rows for contexts of up to n positions: 16 rows
+// of score codes and eight V stages (kernels/prefill_attention_rows.hip)
+uint32_t rows_attention_lds(uint32_t n) { return 16u * ((n + 63u) / 64u * 128u + 32u) + 8u * 2048u; }
+
 int setup_prefill(xpu_qwen3 &e) {
   const xpu_qwen3_config &c = e.c;
   const uint32_t qd = c.heads * c.head_dim;
@@ -466,6 +472,7 @@ int setup_prefill(xpu_qwen3 &e) {
   e.pf_norm_k = e.rt->find_exact("xpu_q3_pf_rmsnorm");
   e.pf_rope_k = e.rt->find_exact("xpu_q3_pf_rope_cache");
   e.pf_attn_k = e.rt->find_exact("xpu_q3_pf_attention");
+  e.pf_attn_rows_k = e.rt->find_exact("xpu_q3_pf_attention_rows");
   e.pf_attn_short_k = e.rt->find_exact("xpu_q3_pf_attention_short");
   const bool common = e.pf_embed_k && e.pf_norm_k && e.pf_rope_k && c.hidden % 8 == 0;
   e.pf_ok = common && e.pf_qkv_k && e.pf_o_k && e.pf_gu_k && e.pf_down_k && e.pf_attn_k &&
@@ -486,9 +493,11 @@ int setup_prefill(xpu_qwen3 &e) {
   e.pf_gemm_ok = common && e.pf_silu_k && e.pf_attn_mfma_k && e.rt->find_exact("xpu_gemm_bf16_nt_dma") &&
                  c.intermediate % 8 == 0 && qd % 8 == 0 && qkv_rows % 8 == 0;
   if (!e.pf_ok && !e.pf_gemm_ok) return XPU_OK;
-  // chunks of 256 positions for the batched GEMV form; up to 4096 for the
-  // GEMM form, whose GEMMs and attention fill the chip only with long chunks
-  e.pf_chunk = e.pf_ok ? std::min<uint32_t>(e.max_seq, 256) : 0;
+  // chunks of 1024 positions for the batched GEMV form (256 leave its
+  // kernels' last blocks alone on the chip: 1531 ids x 2 layers 1681 us,
+  // 1463 with 1024); up to 4096 for the GEMM form, whose GEMMs and attention
+  // fill the chip only with long chunks
+  e.pf_chunk = e.pf_ok ? std::min<uint32_t>(e.max_seq, kBatchedChunk) : 0;
   e.pf_chunk_gemm = e.pf_gemm_ok ? std::min<uint32_t>(e.max_seq, 4096) : 0;
   e.batched_prefill = e.pf_ok;  // the default: the bit-identical form; the GEMM form is opt-in
   return e.pf_ok ? size_prompt_buffers(e, false) : XPU_OK;
@@ -675,6 +684,15 @@ int run_prefill(xpu_qwen3 &e, uint32_t P, bool head) {
         // G = 1 and 2, 1 for G = 4
         const uint32_t qrows = heads / kv == 1 ? 64 : 32, blocks = (T + qrows - 1) / qrows * kv;
         if ((rc = go(e.pf_attn_mfma_k, blocks, 1, 256, 0,
+                     {{8, &e.pf_q}, {8, &kc}, {8, &vc}, {8, &e.pf_a}, {4, &p0}, {4, &T}, {4, &heads}, {4, &kv},
+                      {4, &max_seq}, {4, &scale}})))
+          return rc;
+      } else if (e.pf_attn_rows_k && p0 + T > 128 && p0 + T <= 4096 && rows_attention_lds(p0 + T) <= rt->max_shared) {
+        // 16 queries of a head per block; contexts of one softmax chunk. Up
+        // to 128 positions its fixed cost (one 64-key tile on one wavefront,
+        // ~11 us) exceeds the one-token blocks' (64 ids 11.2 against 7.8 us,
+        // 128 ids 11.7 both, 256 ids 13.6 against 23.4)
+        if ((rc = go(e.pf_attn_rows_k, heads * ((T + 15) / 16), 1, 512, rows_attention_lds(p0 + T),
                      {{8, &e.pf_q}, {8, &kc}, {8, &vc}, {8, &e.pf_a}, {4, &p0}, {4, &T}, {4, &heads}, {4, &kv},
                       {4, &max_seq}, {4, &scale}})))
           return rc;
