@@ -35,11 +35,11 @@ int plan_gemv(const xpu_runtime &rt, int dtype, const void *A, const void *x, ui
   // chunks per batch (6.7 TB/s at 16384^2 fp16, against 5.8-6.2 for 2 rows);
   // shorter rows two per wavefront, 2 chunks per batch, so the bubble at each
   // row's end is shared by two rows (6.6 TB/s at 65536 x 4096 and
-  // 32768 x 8192, against 5.2 and 6.3 for one row). 8 chunks when the vector
-  // is read from global memory, 2 for the 16-bit-load path of unaligned
-  // operands.
-  const bool short_rows = vec && !global_x && K <= 8192;
-  const uint32_t rows = short_rows ? 2 : 1, unroll = !vec ? 2 : global_x ? 8 : short_rows ? 2 : 4;
+  // 32768 x 8192, against 5.2 and 6.3 for one row); the same for operands
+  // that are not 16-byte aligned. 8 chunks when the vector is read from
+  // global memory.
+  const bool short_rows = !global_x && K <= 8192;
+  const uint32_t rows = short_rows ? 2 : 1, unroll = global_x ? 8 : short_rows ? 2 : 4;
   plan.shared = global_x ? 0 : static_cast<uint32_t>(kpad * 2);
   // one block per compute unit, grid-stride over 4-row tiles: each block
   // stages the vector once

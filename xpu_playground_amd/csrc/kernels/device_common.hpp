@@ -17,6 +17,8 @@
 namespace xpu {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// 16 bytes at the alignment of a 16-bit element
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 enum : int { kBf16 = 0, kFp16 = 1 };

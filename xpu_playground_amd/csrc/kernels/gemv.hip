@@ -6,8 +6,8 @@
 // bytes for the staged vector; the grid walks tiles of 4*R rows with a
 // grid-stride loop so each block stages the vector once. Any M, K >= 1 and
 // any leading dimension lda >= K are accepted; the _vec variants need A, x
-// 16-byte aligned and K, lda multiples of 8 (the host checks), the others
-// use 16-bit loads. The _vecg variants read the vector from global memory
+// 16-byte aligned and K, lda multiples of 8 (the host checks), the _any
+// variants load 16 bytes at any element. The _vecg variants read the vector from global memory
 // when it does not fit in LDS.
 #include "gemv_core.hpp"
 
@@ -56,11 +56,11 @@ XPU_DEVICE void gemv_entry(const uint16_t *__restrict__ A, const uint16_t *__res
 // 512-column chunks per pipelined load batch
 #define XPU_GEMV_TYPES(R, U)                                                         \
   XPU_GEMV_VARIANT(xpu_gemv_bf16_r##R##u##U##_vec, xpu::kBf16, R, U, true, false)   \
-  XPU_GEMV_VARIANT(xpu_gemv_fp16_r##R##u##U##_vec, xpu::kFp16, R, U, true, false)
+  XPU_GEMV_VARIANT(xpu_gemv_fp16_r##R##u##U##_vec, xpu::kFp16, R, U, true, false)   \
+  XPU_GEMV_VARIANT(xpu_gemv_bf16_r##R##u##U##_any, xpu::kBf16, R, U, false, false)  \
+  XPU_GEMV_VARIANT(xpu_gemv_fp16_r##R##u##U##_any, xpu::kFp16, R, U, false, false)
 
 XPU_GEMV_TYPES(1, 4)
 XPU_GEMV_TYPES(2, 2)
-XPU_GEMV_VARIANT(xpu_gemv_bf16_r1u2_any, xpu::kBf16, 1, 2, false, false)
-XPU_GEMV_VARIANT(xpu_gemv_fp16_r1u2_any, xpu::kFp16, 1, 2, false, false)
 XPU_GEMV_VARIANT(xpu_gemv_bf16_r1u8_vecg, xpu::kBf16, 1, 8, true, true)
 XPU_GEMV_VARIANT(xpu_gemv_fp16_r1u8_vecg, xpu::kFp16, 1, 8, true, true)

@@ -42,8 +42,8 @@ XPU_DEVICE void stage_vector(uint16_t *xs, const uint16_t *__restrict__ x, uint3
   }
   for (uint32_t i = threadIdx.x * 8u; i < kpad; i += threads * 8u) {
     u32x4 v;
-    if (VEC && i + 8u <= K) {
-      v = *reinterpret_cast<const u32x4 *>(x + i);
+    if (i + 8u <= K) {
+      v = *reinterpret_cast<const u32x4_any *>(x + i);
     } else {
       uint32_t w[8];
 #pragma unroll
@@ -55,18 +55,32 @@ XPU_DEVICE void stage_vector(uint16_t *xs, const uint16_t *__restrict__ x, uint3
   }
 }
 
-// 8 codes of row starting at p, columns col..col+7 of a row of length K.
-template <bool VEC>
-XPU_DEVICE u32x4 load_row8(const uint16_t *__restrict__ p, uint32_t col, uint32_t K) {
-  if constexpr (VEC) {
-    return load_nt16(p);
-  } else {
-    uint32_t w[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) w[e] = (col + e < K) ? __builtin_nontemporal_load(p + e) : 0u;
-    return u32x4{w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16),
-                 w[6] | (w[7] << 16)};
+// 8 codes (16 bytes) of a row at p. Rows that are not 16-byte aligned are
+// read with the same 16-byte loads (global memory runs in unaligned access
+// mode on gfx950): 5003 x 3001 bf16 with a pitch of 3005, 51.1 us with eight
+// 2-byte loads instead.
+template <bool VEC> XPU_DEVICE u32x4 load_row8(const uint16_t *__restrict__ p) {
+  if constexpr (VEC) return load_nt16(p);
+  else return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any *>(p));
+}
+
+// The codes of columns col .. col + 7 (zeros past K) for col < K, from the 8
+// codes at column min(col, K - 8): the lane whose slice crosses K shifts the
+// codes before its own out.
+XPU_DEVICE u32x4 cut_tail(const u32x4 &v, uint32_t col, uint32_t K) {
+  const uint32_t s = col + 8u > K && col < K ? (col + 8u - K) * 16u : 0u;  // bits
+  uint64_t lo = v.x | (static_cast<uint64_t>(v.y) << 32), hi = v.z | (static_cast<uint64_t>(v.w) << 32);
+  if (s >= 64u) {
+    lo = hi;
+    hi = 0;
   }
+  const uint32_t q = s & 63u;
+  if (q) {
+    lo = (lo >> q) | (hi << (64u - q));
+    hi >>= q;
+  }
+  return u32x4{static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi),
+               static_cast<uint32_t>(hi >> 32)};
 }
 
 template <int DT, int R>
@@ -102,14 +116,12 @@ XPU_DEVICE void gemv_row_ptrs(const uint16_t *__restrict__ A, uint64_t lda, uint
 }
 
 template <int R, int U, bool VEC>
-XPU_DEVICE void gemv_load_batch(u32x4 (&buf)[U][R], const uint16_t *const (&rows)[R], uint32_t j0,
-                                uint32_t K) {
-  const uint32_t lane = lane_id();
+XPU_DEVICE void gemv_load_batch(u32x4 (&buf)[U][R], const uint16_t *const (&rows)[R], uint32_t j0) {
 #pragma unroll
   for (int u = 0; u < U; ++u)
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      buf[u][r] = load_row8<VEC>(rows[r] + (j0 + u) * 512u, (j0 + u) * 512u + lane * 8u, K);
+      buf[u][r] = load_row8<VEC>(rows[r] + (j0 + u) * 512u);
 }
 
 // Canonical dot products of R rows (see gemv_row_ptrs) with the staged
@@ -135,12 +147,31 @@ XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, ui
   // pipelined: the loads of batch j + U are issued before the FMAs of batch
   // j, and a scheduling barrier keeps the compiler from interleaving each
   // load with its use (which would leave one load in flight per wave).
-  auto load_batch = [&](u32x4 (&buf)[U][R], uint32_t j0) { gemv_load_batch<R, U, VEC>(buf, rows, j0, K); };
+  auto load_batch = [&](u32x4 (&buf)[U][R], uint32_t j0) { gemv_load_batch<R, U, VEC>(buf, rows, j0); };
   auto fma_batch = [&](const u32x4 (&buf)[U][R], uint32_t j0) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
       fma_chunk<DT, R>(acc, buf[u], *reinterpret_cast<const u32x4 *>(xl + (j0 + u) * 512u));
   };
+  // With two-chunk batches (short rows) the chunk that crosses K and the full
+  // chunk left over after the batches are loaded ahead of them, so that a row
+  // does not wait for its end on its own. Long rows load them where they are
+  // used: the loads ahead of the first batch cost 16384^2 fp16 5%. A row of
+  // fewer than 8 columns has no 8 codes to load.
+  constexpr bool kEarly = U == 2;
+  const uint32_t tail_col = nfull * 512u + lane * 8u;
+  const bool tail8 = K % 512u != 0 && K >= 8u, spare = kEarly && nfull % 2u != 0;
+  u32x4 tail[R], over[R];
+  auto load_tail = [&]() {
+    const uint32_t at = tail_col < K - 8u ? tail_col : K - 8u;
+#pragma unroll
+    for (int r = 0; r < R; ++r) tail[r] = load_row8<VEC>(rows[r] + static_cast<int32_t>(at - lane * 8u));
+  };
+  if (kEarly && tail8) load_tail();
+  if (spare) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) over[r] = load_row8<VEC>(rows[r] + (nfull - 1u) * 512u);
+  }
   uint32_t j = 0;
   if (nfull >= static_cast<uint32_t>(U)) {
     u32x4 b0[U][R], b1[U][R];
@@ -165,20 +196,40 @@ XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, ui
       j += U;
     }
   }
-  for (; j < nfull; ++j) {
-    u32x4 a[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) a[r] = load_row8<VEC>(rows[r] + j * 512u, j * 512u + lane * 8u, K);
-    fma_chunk<DT, R>(acc, a, *reinterpret_cast<const u32x4 *>(xl + j * 512u));
+  if (spare) {
+    fma_chunk<DT, R>(acc, over, *reinterpret_cast<const u32x4 *>(xl + j * 512u));
+    ++j;
   }
-  if (K % 512u) {
-    const uint32_t col = nfull * 512u + lane * 8u;
-    if (col < K) {
+  if constexpr (!kEarly)
+    for (; j < nfull; ++j) {
       u32x4 a[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) a[r] = load_row8<VEC>(rows[r] + nfull * 512u, col, K);
+      for (int r = 0; r < R; ++r) a[r] = load_row8<VEC>(rows[r] + j * 512u);
+      fma_chunk<DT, R>(acc, a, *reinterpret_cast<const u32x4 *>(xl + j * 512u));
+    }
+  if constexpr (VEC && !kEarly) {
+    if (K % 512u && tail_col < K) {
+      u32x4 a[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) a[r] = load_row8<true>(rows[r] + nfull * 512u);
       fma_chunk<DT, R>(acc, a, *reinterpret_cast<const u32x4 *>(xl + nfull * 512u));
     }
+  } else if (K % 512u) {
+    u32x4 a[R];
+    if (tail8) {
+      if (!kEarly) load_tail();
+#pragma unroll
+      for (int r = 0; r < R; ++r) a[r] = VEC ? tail[r] : cut_tail(tail[r], tail_col, K);
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        uint32_t w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[e] = tail_col + e < K ? rows[r][e] : 0u;
+        a[r] = u32x4{w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16)};
+      }
+    }
+    if (tail_col < K) fma_chunk<DT, R>(acc, a, *reinterpret_cast<const u32x4 *>(xl + nfull * 512u));
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) out[r] = wave_butterfly(fold8(acc[r]));

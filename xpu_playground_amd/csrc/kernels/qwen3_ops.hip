@@ -177,7 +177,7 @@ XPU_DEVICE void fused_gemv(const uint16_t *__restrict__ W, uint32_t units, uint3
   if (base + wave * per_wave < units && K / 512u >= static_cast<uint32_t>(U)) {
     const uint16_t *rows[R];
     xpu::gemv_row_ptrs<R, PAIRED>(W, K, rows_total, base + wave * per_wave, pair_offset, rows);
-    xpu::gemv_load_batch<R, U, true>(first, rows, 0, K);
+    xpu::gemv_load_batch<R, U, true>(first, rows, 0);
     have_first = true;
   }
   prologue();
