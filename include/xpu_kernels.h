@@ -40,15 +40,18 @@ int xpu_gemv(xpu_runtime *rt, int dtype, const void *A, const void *x, void *y,
  * or 128x128) is the one with the least estimated time at this shape on this
  * GPU's compute units (xpu_gemm_tile). Any M, N, K and 2-byte aligned
  * pointers: the operands are read in place (the reference pads them on the
- * host, gemm.cpp:75-85). Outputs that leave most compute units idle even
- * with 128 x 128 tiles, with 8 or more 64-deep K-slices, split K over the
- * idle units (FP32 partials in the runtime's workspace, added in split
- * order). Asynchronous on the runtime's stream. */
+ * host, gemm.cpp:75-85). Outputs for which that tile leaves compute units
+ * idle are run in 64x128 or 32x128 tiles of the same sums where that is
+ * faster; those that leave most units idle even with 128 x 128 tiles, with 8
+ * or more 64-deep K-slices, may split K over the idle units (FP32 partials
+ * in the runtime's workspace, added in split order). Asynchronous on the
+ * runtime's stream. */
 int xpu_gemm(xpu_runtime *rt, int dtype, const void *A, const void *B, void *C,
              uint32_t M, uint32_t N, uint32_t K);
 
-/* The block tile xpu_gemm uses for an M x N output on this runtime's GPU:
- * *rows x *cols. No device work. The reference's counterpart is the
+/* The block tile, of the four, that xpu_gemm chooses for an M x N output on
+ * this runtime's GPU (before any smaller tile for idle units, which depends
+ * on K too): *rows x *cols. No device work. The reference's counterpart is the
  * large_tile expression of gemm.cpp:145. */
 int xpu_gemm_tile(const xpu_runtime *rt, uint32_t M, uint32_t N, uint32_t *rows, uint32_t *cols);
 
@@ -58,12 +61,13 @@ int xpu_gemm_tile(const xpu_runtime *rt, uint32_t M, uint32_t N, uint32_t *rows,
 /* xpu_gemm without allocation. No counterpart in the reference: for callers
  * that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc). Same kernels and results
- * as xpu_gemm, bit for bit. Where xpu_gemm splits K (outputs that leave most
- * compute units idle, with 8 or more 64-deep K-slices), its FP32 partials
- * (splits x M x round_up(N, 4) x 4 bytes) go into a fixed device array of
- * XPU_GEMM_NOALLOC_SCRATCH_BYTES per GPU, set up when the first runtime on
- * that GPU is created and held until the process ends, instead of the
- * runtime's workspace; other shapes use no scratch. Needs above the array
+ * as xpu_gemm, bit for bit. Where xpu_gemm may split K (outputs that leave
+ * most compute units idle, with 8 or more 64-deep K-slices), its FP32
+ * partials (splits x M x round_up(N, 4) x 4 bytes) go into a fixed device
+ * array of XPU_GEMM_NOALLOC_SCRATCH_BYTES per GPU, set up when the first
+ * runtime on that GPU is created and held until the process ends, instead of
+ * the runtime's workspace; other shapes use no scratch. Shapes whose largest
+ * number of splits would need more than the array
  * fail with XPU_ERR_INVALID before any launch. Calls no hipMalloc/hipFree.
  * All calls on one GPU share the array: calls that overlap on one GPU (other
  * streams or runtimes) race. */

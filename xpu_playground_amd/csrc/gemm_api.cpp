@@ -44,24 +44,100 @@ constexpr GemmTile kTiles[] = {{"", 256, 256, 1, 1.0, 0.0, true, true},
 // (4096^3), 224 x 256 takes outputs where it still does and cuts each unit's
 // work by 1/8 (3000 x 4097: 238 blocks instead of 204), and outputs that
 // leave most compute units idle take a smaller one.
+uint64_t tile_count(uint64_t M, uint64_t N, uint32_t rows, uint32_t cols) {
+  return ((M + rows - 1) / rows) * ((N + cols - 1) / cols);
+}
+
+double tile_cost(const GemmTile &t, uint32_t compute_units, uint32_t M, uint32_t n_cols) {
+  const uint64_t w = (tile_count(M, n_cols, t.rows, t.cols) + compute_units - 1) / std::max(1u, compute_units);
+  const double area = static_cast<double>(t.rows) * t.cols;
+  return t.per_cu == 2 ? static_cast<double>(w / 2) * 2.0 * area / t.pair_rate +
+                             static_cast<double>(w % 2) * area / t.solo_rate
+                       : static_cast<double>(w) * area / t.solo_rate;
+}
+
 const GemmTile &choose_tile(uint32_t compute_units, uint32_t M, uint32_t n_cols, bool nt = false) {
   const GemmTile *best = &kTiles[0];
   double best_cost = 0;
   for (const GemmTile &t : kTiles) {
     if (nt && !t.nt_forms) continue;
-    const uint64_t tiles = ((static_cast<uint64_t>(M) + t.rows - 1) / t.rows) *
-                           ((static_cast<uint64_t>(n_cols) + t.cols - 1) / t.cols);
-    const uint64_t w = (tiles + compute_units - 1) / std::max(1u, compute_units);
-    const double area = static_cast<double>(t.rows) * t.cols;
-    const double cost = t.per_cu == 2 ? static_cast<double>(w / 2) * 2.0 * area / t.pair_rate +
-                                            static_cast<double>(w % 2) * area / t.solo_rate
-                                      : static_cast<double>(w) * area / t.solo_rate;
+    const double cost = tile_cost(t, compute_units, M, n_cols);
     if (&t == &kTiles[0] || cost < best_cost) {
       best = &t;
       best_cost = cost;
     }
   }
   return *best;
+}
+
+// The most ranges xpu_gemm cuts K into (1: whole K): where 128 x 128 tiles
+// leave at least half the compute units idle, about CUs / tiles ranges of a
+// multiple of 2 slices, for K of 24 slices or more or partials of at most
+// 4 MiB (1024^3, 16 slices and 16 MB of partials, is slower split at any
+// tile: 12.8 us against 6.7).
+uint32_t max_splits(uint32_t compute_units, const GemmTile &tile, uint32_t M, uint32_t N, uint32_t K) {
+  const uint64_t tiles = tile_count(M, N, 128, 128);
+  const uint32_t slices = (K + 63) / 64;
+  if (tile.rows != 128 || tile.cols != 128 || tiles * 2 > compute_units || slices < 8) return 1;
+  const uint32_t want = static_cast<uint32_t>((compute_units + tiles - 1) / tiles);
+  const uint32_t spl = ((slices + want - 1) / want + 1) / 2 * 2, splits = (slices + spl - 1) / spl;
+  const uint64_t bytes = static_cast<uint64_t>(splits) * M * ((N + 3) / 4 * 4) * 4;
+  return splits >= 2 && (slices >= 24 || bytes <= (4ull << 20)) ? splits : 1;
+}
+
+// The small tiles (kernels/gemm.hip): stages
+// (slices per group) and us per 64-deep slice with w blocks on the busiest
+// unit, w * pair_us for w >= 2.
+struct SmallTile {
+  const char *tag;
+  uint32_t rows, cols, stages;
+  double solo_us, pair_us;
+};
+constexpr SmallTile kSmallTiles[] = {{"_m32", 32, 128, 4, 0.26, 0.27}, {"_m64", 64, 128, 3, 0.33, 0.36}};
+
+struct SmallPlan {
+  const SmallTile *tile = nullptr;  // null: the tile of choose_tile, whole K
+  uint64_t tiles = 0;
+  uint32_t splits = 1, slices = 0;  // K ranges, and slices per range
+};
+
+// A small tile, with K whole or in up to `limit` ranges, where its estimated
+// time is below the chosen tile's: us per slice (a group of slices past K
+// costs as much) over the busiest unit's blocks, plus for a split the second
+// launch (2 us), each range's load in the reduction (0.12 us) and the
+// partials' round trip (0.55 us per MB). Fitted to 19 swept shapes, bf16 and
+// back to back: it takes the measured fastest plan or one within 8% of it.
+// Against 128 x 128 tiles, K split as max_splits says: 24 x 4096 x 4096 (8
+// ranges of 32 x 128) 12.0 -> 9.1 us, 64 x 1024 x 4096 13.1 -> 8.1, 512^3
+// (whole K) 8.9 -> 4.3, 1024^3 9.5 -> 6.7, 300 x 3000 x 3000 20.5 -> 17.3,
+// 1500 x 1000 x 600 (64 x 128) 7.7 -> 6.6; 2048 x 2048 x 512 stays (8.0
+// against 9.0).
+SmallPlan choose_small(uint32_t compute_units, const GemmTile &tile, uint32_t M, uint32_t N, uint32_t K,
+                       uint32_t limit) {
+  SmallPlan plan;
+  if (tile.rows > 128) return plan;
+  const uint32_t slices = (K + 63) / 64, cus = std::max(1u, compute_units);
+  // 0.375 us is a slice's share of 128 x 128 outputs at the large tile's rate
+  double best = tile_cost(tile, cus, M, N) / (128 * 128) * 0.375 * slices;
+  const double mb = static_cast<double>(M) * ((N + 3) / 4 * 4) * 4e-6;
+  for (const SmallTile &t : kSmallTiles) {
+    const uint64_t tiles = tile_count(M, N, t.rows, t.cols);
+    // as many ranges as fill the units, then fewer, halving
+    for (uint32_t want = static_cast<uint32_t>(std::min<uint64_t>(limit, std::max<uint64_t>(1, cus / tiles)));;
+         want /= 2) {
+      const uint32_t per = ((slices + want - 1) / want + t.stages - 1) / t.stages * t.stages;
+      const uint32_t splits = (slices + per - 1) / per;
+      const uint64_t w = (tiles * splits + cus - 1) / cus;
+      const double us = per * (w == 1 ? t.solo_us : static_cast<double>(w) * t.pair_us) +
+                        (splits >= 2 ? 2.0 + splits * (0.12 + 0.55 * mb) : 0.0);
+      if (us < best) {
+        best = us;
+        plan = {&t, tiles, splits, per};
+      }
+      if (want <= 1) break;
+    }
+  }
+  return plan;
 }
 
 }  // namespace
@@ -92,50 +168,44 @@ int gemm_run(xpu_runtime *rt, int dtype, const void *A, const void *B, void *C, 
   // operands' ends (kernels/gemm.hip)
   const bool edge = K % 8 != 0 || N % 2 != 0;
   const char *dt = dtype ? "fp16" : "bf16";
-  // Split K where even 128 x 128 tiles leave at least half the compute
-  // units idle and the reduction is long enough to pay for the partials'
-  // round trip: about CUs / tiles ranges of a multiple of 2 slices; FP32
-  // partials [split][M][pitch] in the workspace (the runtime's, or the
-  // caller's fixed array), then one reduction in split order that rounds to
-  // the output type. Within the GEMM's tolerance, not bit-equal to one
-  // chain (the FP32 sum is re-associated at the range boundaries). Measured
-  // against whole-K 128 x 128 tiles (bf16): 1024 x 1024 x 4096 42.6 -> 23.0
-  // us, 768 x 768 x 8192 82.5 -> 26.9, 512^3 12.1 -> 9.2, but 1024^3 (16
-  // slices, 16 MB of partials) 12.5 -> 17.9: so K of 24 slices or more, or
-  // partials of at most 4 MiB.
-  {
-    const uint64_t t128 = ((static_cast<uint64_t>(M) + 127) / 128) * ((static_cast<uint64_t>(N) + 127) / 128);
-    const uint32_t nslices = (K + 63) / 64;
-    if (std::string(tile.tag) == "_t128" && t128 * 2 <= rt->compute_units && nslices >= 8) {
-      const uint32_t want = static_cast<uint32_t>((rt->compute_units + t128 - 1) / t128);
-      const uint32_t spl = ((nslices + want - 1) / want + 1) / 2 * 2, splits = (nslices + spl - 1) / spl;
-      const uint32_t pitch = (N + 3) / 4 * 4;
-      const uint64_t bytes = static_cast<uint64_t>(splits) * M * pitch * 4;
-      if (splits >= 2 && (nslices >= 24 || bytes <= (4ull << 20))) {
-        void *ws = fixed_workspace;
-        int rc = XPU_OK;
-        if (!ws) rc = rt->scratch(bytes, &ws);
-        else if (bytes > fixed_capacity)
-          rc = set_error(XPU_ERR_INVALID, "xpu_gemm_noalloc: the split-K partials need " + std::to_string(bytes) +
-                                              " bytes, above the " + std::to_string(fixed_capacity) +
-                                              "-byte scratch array");
-        if (rc) return rc;
-        const std::string pname = std::string("xpu_gemm_") + dt + "_t128_part_dma" + (edge ? "_edge" : "");
-        const xpu::KernelInfo *kp = rt->find_exact(pname);
-        const xpu::KernelInfo *kr = rt->find_exact("xpu_gemm_splitk_reduce_any");
-        if (!kp || !kr) return set_error(XPU_ERR_NOT_FOUND, "kernel is absent from module: " + pname);
-        uint32_t kb = spl, ldp = pitch, n_out = N;
-        const xpu_kernel_arg pargs[] = {{8, &a_use}, {8, &b_use}, {8, &ws},  {4, &M},     {4, &n_run},
-                                        {4, &k_run}, {4, &kb},    {4, &ldp}, {4, &n_out}};
-        if ((rc = rt->launch(*kp, static_cast<uint32_t>(t128 * splits), 1, 256, 0, pargs, 9))) return rc;
-        const uint64_t threads = static_cast<uint64_t>(M) * ((N + 3) / 4);
-        const uint32_t grid =
-            static_cast<uint32_t>(std::min<uint64_t>((threads + 255) / 256, rt->compute_units * 8ull));
-        uint32_t ldc = N, ns = splits, d = static_cast<uint32_t>(dtype);
-        const xpu_kernel_arg rargs[] = {{8, &ws}, {8, &C}, {4, &M}, {4, &n_run}, {4, &ldp}, {4, &ldc}, {4, &ns}, {4, &d}};
-        return rt->launch(*kr, grid, 1, 256, 0, rargs, 8);
-      }
+  // Where K may be split, the FP32 partials [split][M][pitch] go into the
+  // workspace (the runtime's, or the caller's fixed array) and one reduction
+  // in split order rounds to the output type. Within the GEMM's tolerance,
+  // not bit-equal to one chain (the FP32 sum is re-associated at the range
+  // boundaries). The fixed array's limit is stated on max_splits' partials,
+  // which no plan exceeds, so that the accepted shapes do not depend on the
+  // tile a plan takes.
+  const uint32_t pitch = (N + 3) / 4 * 4;
+  const uint64_t split_bytes = static_cast<uint64_t>(M) * pitch * 4;
+  const uint32_t limit = max_splits(rt->compute_units, tile, M, N, K);
+  if (fixed_workspace && limit >= 2 && limit * split_bytes > fixed_capacity)
+    return set_error(XPU_ERR_INVALID, "xpu_gemm_noalloc: the split-K partials need " +
+                                          std::to_string(limit * split_bytes) + " bytes, above the " +
+                                          std::to_string(fixed_capacity) + "-byte scratch array");
+  if (const SmallPlan plan = choose_small(rt->compute_units, tile, M, N, K, limit); plan.tile) {
+    const std::string stem = std::string("xpu_gemm_") + dt + plan.tile->tag;
+    const bool part = plan.splits >= 2;
+    const std::string name = stem + (part ? "_part_dma" : c16 ? "_dma" : "_dmau") + (edge ? "_edge" : "");
+    const xpu::KernelInfo *k = rt->find_exact(name);
+    const xpu::KernelInfo *kr = part ? rt->find_exact("xpu_gemm_splitk_reduce_any") : nullptr;
+    if (!k || (part && !kr)) return set_error(XPU_ERR_NOT_FOUND, "kernel is absent from module: " + name);
+    void *out = C;
+    uint32_t kb = K, ld_out = N, n_out = N;
+    int rc = XPU_OK;
+    if (part) {
+      out = fixed_workspace;
+      if (!out && (rc = rt->scratch(plan.splits * split_bytes, &out))) return rc;
+      kb = plan.slices;
+      ld_out = pitch;
     }
+    const xpu_kernel_arg args[] = {{8, &a_use}, {8, &b_use}, {8, &out},    {4, &M},    {4, &n_run},
+                                   {4, &k_run}, {4, &kb},    {4, &ld_out}, {4, &n_out}};
+    if ((rc = rt->launch(*k, static_cast<uint32_t>(plan.tiles * plan.splits), 1, 256, 0, args, 9)) || !part) return rc;
+    const uint64_t threads = static_cast<uint64_t>(M) * (pitch / 4);
+    const uint32_t grid = static_cast<uint32_t>(std::min<uint64_t>((threads + 255) / 256, rt->compute_units * 8ull));
+    uint32_t ldc = N, ns = plan.splits, d = static_cast<uint32_t>(dtype);
+    const xpu_kernel_arg rargs[] = {{8, &out}, {8, &C}, {4, &M}, {4, &n_run}, {4, &ld_out}, {4, &ldc}, {4, &ns}, {4, &d}};
+    return rt->launch(*kr, grid, 1, 256, 0, rargs, 8);
   }
   // the 256 x 256 and 224 x 256 kernels come in a form for an odd number (3
   // or more) of 64-deep K-slices, which skips the slice of zeros that closes

@@ -3,8 +3,8 @@
 // gemm_kernel.hpp:25-143, argument order (a, b, c, m, n, k) of
 // level_zero/gem_spv_entry.cpp:28-60).
 //
-// Block tile (64 MI) x (64 NJ), K-slice BK (64 or 32), two LDS stages, 256
-// threads: four wavefronts in a 2 x 2 arrangement, each owning 32 MI x 32 NJ
+// Block tile (64 MI) x (64 NJ), K-slice BK (64 or 32), two LDS stages (the small
+// tiles: three or four), 256 threads: four wavefronts in a 2 x 2 arrangement, each owning 32 MI x 32 NJ
 // of C as MI x NJ tiles of v_mfma_f32_32x32x16_{bf16,f16}. The large tile is
 // 256 x 256 (MI = NJ = 4, 256 FP32 accumulators per lane). The small tiles,
 // 128 x 256 (the reference's small tile, gemm_kernel.hpp:26-27) and
@@ -593,7 +593,7 @@ XPU_DEVICE void body(const uint16_t *__restrict__ A, const uint16_t *__restrict_
     // Rows of the band in batches of kBatch read-back rows: every LDS read of
     // a batch is issued before the first conversion. Bands inside M x n_out
     // skip the per-row bounds checks.
-    constexpr uint32_t kBatch = 4;
+    constexpr uint32_t kBatch = MI % 2 && 32u / kRpr < 4u ? 32u / kRpr : 4u;
     static_assert((64u / kRpr) % kBatch == 0 && (MI % 2 == 0 || (32u / kRpr) % kBatch == 0),
                   "whole batches in every band");
     const uint32_t iters = band_rows / kRpr;
@@ -753,6 +753,7 @@ extern "C" __global__ __launch_bounds__(256) void xpu_gemm_splitk_reduce(const f
 extern "C" __global__ __launch_bounds__(256) void xpu_gemm_splitk_reduce_any(
     const float *__restrict__ P, uint16_t *__restrict__ C, uint32_t M, uint32_t N, uint32_t pitch, uint32_t ldc,
     uint32_t splits, uint32_t dtype) {
+  constexpr uint32_t kBatch = 7;  // splits loaded ahead of their additions
   const uint32_t groups = (N + 3u) / 4u;
   const uint64_t total = static_cast<uint64_t>(M) * groups, split4 = static_cast<uint64_t>(M) * pitch / 4u;
   for (uint64_t g = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; g < total;
@@ -760,15 +761,27 @@ extern "C" __global__ __launch_bounds__(256) void xpu_gemm_splitk_reduce_any(
     const uint32_t m = static_cast<uint32_t>(g / groups), n = static_cast<uint32_t>(g % groups) * 4u;
     const float4 *p = reinterpret_cast<const float4 *>(P + static_cast<uint64_t>(m) * pitch + n);
     float4 acc = p[0];
-    for (uint32_t s = 1; s < splits; ++s) {
-      const float4 v = p[s * split4];
-      acc = float4{acc.x + v.x, acc.y + v.y, acc.z + v.z, acc.w + v.w};
+    for (uint32_t s0 = 1; s0 < splits; s0 += kBatch) {
+      float4 v[kBatch];
+#pragma unroll
+      for (uint32_t k = 0; k < kBatch; ++k) v[k] = p[min(s0 + k, splits - 1u) * split4];
+#pragma unroll
+      for (uint32_t k = 0; k < kBatch; ++k)
+        if (s0 + k < splits) acc = float4{acc.x + v[k].x, acc.y + v[k].y, acc.z + v[k].z, acc.w + v[k].w};
     }
     const float y[4] = {acc.x, acc.y, acc.z, acc.w};
     uint16_t *dst = C + static_cast<uint64_t>(m) * ldc + n;
+    uint32_t c[4];
 #pragma unroll
-    for (uint32_t e = 0; e < 4; ++e)
-      if (n + e < N) dst[e] = static_cast<uint16_t>(dtype ? xpu::f32_to_fp16(y[e]) : xpu::f32_to_bf16(y[e]));
+    for (uint32_t e = 0; e < 4; ++e) c[e] = dtype ? xpu::f32_to_fp16(y[e]) : xpu::f32_to_bf16(y[e]);
+    if (n + 4u <= N) {
+      const xpu::u32x2 w{c[0] | (c[1] << 16), c[2] | (c[3] << 16)};
+      __builtin_memcpy(dst, &w, 8);  // 2-byte aligned: unaligned access mode on gfx950
+    } else {
+#pragma unroll
+      for (uint32_t e = 0; e < 3; ++e)
+        if (n + e < N) dst[e] = static_cast<uint16_t>(c[e]);
+    }
   }
 }
 
@@ -900,21 +913,45 @@ XPU_GEMM_DMA_VARIANT(xpu_gemm_bf16_t128_dmau, xpu::kBf16, 2, 2, 64, 2, 2, 2, 2, 
 XPU_GEMM_DMA_VARIANT(xpu_gemm_fp16_t128_dmau, xpu::kFp16, 2, 2, 64, 2, 2, 2, 2, false, false)
 
 // Split K for [k][n] products that leave most compute units idle even with
-// 128 x 128 tiles (a small output with a long reduction): FP32 partials of
-// each K range (kb slices, a multiple of 2), added by
+// small tiles (a small output with a long reduction): FP32 partials of
+// each K range (kb slices, a multiple of the stages), added by
 // xpu_gemm_splitk_reduce_any; _edge as for the whole-K kernels.
-#define XPU_GEMM_PART_KN(NAME, DT, EDGE)                                                                   \
-  extern "C" __global__ __launch_bounds__(256, 2) void NAME(                                               \
+#define XPU_GEMM_PART_KN(NAME, DT, MI, NJ, S, P, MINB, EDGE, WN)                                           \
+  extern "C" __global__ __launch_bounds__(256, MINB) void NAME(                                            \
       const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, uint16_t *__restrict__ C, uint32_t M, \
       uint32_t N, uint32_t K, uint32_t kb, uint32_t ldc, uint32_t n_out) {                                  \
     XPU_STAMP(xpu::kStampGemm);                                                                             \
-    xpu::dma::body<DT, 2, 2, 64, 2, 2, 2, true, false, false, false, true, EDGE>(A, B, C, M, N, K, kb, ldc, \
-                                                                                n_out);                    \
+    xpu::dma::body<DT, MI, NJ, 64, S, P, 2, true, false, false, false, true, EDGE, WN>(A, B, C, M, N, K, kb, \
+                                                                                      ldc, n_out);         \
   }
-XPU_GEMM_PART_KN(xpu_gemm_bf16_t128_part_dma, xpu::kBf16, false)
-XPU_GEMM_PART_KN(xpu_gemm_bf16_t128_part_dma_edge, xpu::kBf16, true)
-XPU_GEMM_PART_KN(xpu_gemm_fp16_t128_part_dma, xpu::kFp16, false)
-XPU_GEMM_PART_KN(xpu_gemm_fp16_t128_part_dma_edge, xpu::kFp16, true)
+
+// Small tiles for outputs that leave compute units idle or half loaded at
+// 128 x 128: 32 x 128 (1 x 4 wavefronts of 32 x 32, four stages of 20 KiB)
+// and 64 x 128 (2 x 2 wavefronts of 32 x 64, three stages of 24 KiB). A wavefront's slice is 4 or 8 MFMAs, far below
+// the latency of the next slice's loads, so these blocks are bound by the
+// latency of their slice chain: 0.26 and 0.33 us per 64-deep slice (128 x
+// 128 with two stages: 0.62), which is also why deeper rings pay: with two
+// slices in flight 64 x 128 keeps two blocks per unit, where four stages
+// (one block) gave 12.8 against 13.0 us at 1024 x 2048 x 2048 but 10.1
+// against 9.0 at 2048 x 2048 x 512; six stages of 32 x 128 were slower
+// (1024^3 7.4 us against 6.7). The same k-order per MFMA chain as the other
+// tiles: the same bits. bf16, back to back, against 128 x 128: 1024^3 9.5 ->
+// 6.7 us, 512^3 6.0 -> 4.3, 1024 x 2048 x 2048 22.5 -> 13.0.
+#define XPU_GEMM_SMALL(TAG, MI, NJ, S, P, MINB, WN)                                                                 \
+  XPU_GEMM_DMA_VARIANT1(xpu_gemm_bf16##TAG##_dma, xpu::kBf16, MI, NJ, 64, S, P, 2, MINB, true, false, false, WN)       \
+  XPU_GEMM_DMA_VARIANT1(xpu_gemm_bf16##TAG##_dma_edge, xpu::kBf16, MI, NJ, 64, S, P, 2, MINB, true, false, true, WN)   \
+  XPU_GEMM_DMA_VARIANT1(xpu_gemm_bf16##TAG##_dmau, xpu::kBf16, MI, NJ, 64, S, P, 2, MINB, false, false, false, WN)     \
+  XPU_GEMM_DMA_VARIANT1(xpu_gemm_bf16##TAG##_dmau_edge, xpu::kBf16, MI, NJ, 64, S, P, 2, MINB, false, false, true, WN) \
+  XPU_GEMM_PART_KN(xpu_gemm_bf16##TAG##_part_dma, xpu::kBf16, MI, NJ, S, P, MINB, false, WN)                        \
+  XPU_GEMM_PART_KN(xpu_gemm_bf16##TAG##_part_dma_edge, xpu::kBf16, MI, NJ, S, P, MINB, true, WN)                    \
+  XPU_GEMM_DMA_VARIANT1(xpu_gemm_fp16##TAG##_dma, xpu::kFp16, MI, NJ, 64, S, P, 2, MINB, true, false, false, WN)       \
+  XPU_GEMM_DMA_VARIANT1(xpu_gemm_fp16##TAG##_dma_edge, xpu::kFp16, MI, NJ, 64, S, P, 2, MINB, true, false, true, WN)   \
+  XPU_GEMM_DMA_VARIANT1(xpu_gemm_fp16##TAG##_dmau, xpu::kFp16, MI, NJ, 64, S, P, 2, MINB, false, false, false, WN)     \
+  XPU_GEMM_DMA_VARIANT1(xpu_gemm_fp16##TAG##_dmau_edge, xpu::kFp16, MI, NJ, 64, S, P, 2, MINB, false, false, true, WN) \
+  XPU_GEMM_PART_KN(xpu_gemm_fp16##TAG##_part_dma, xpu::kFp16, MI, NJ, S, P, MINB, false, WN)                        \
+  XPU_GEMM_PART_KN(xpu_gemm_fp16##TAG##_part_dma_edge, xpu::kFp16, MI, NJ, S, P, MINB, true, WN)
+XPU_GEMM_SMALL(_m32, 1, 1, 4, 0, 1, 4)
+XPU_GEMM_SMALL(_m64, 1, 2, 3, 1, 2, 2)
 
 // dst[r][c] = src[r * src_ld + c] for c < cols, 0 for cols <= c < dst_cols
 // (dst_cols % 8 == 0, dst 16-byte aligned): the zero padding of the
