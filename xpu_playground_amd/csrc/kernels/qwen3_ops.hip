@@ -21,6 +21,8 @@
 // position contiguous).
 #include "qwen3_core.hpp"
 
+#include <type_traits>
+
 using xpu::u32x4;
 
 // ------------------------------------------------------------ reference entries
@@ -918,23 +920,33 @@ extern "C" __global__ __launch_bounds__(256) void xpu_q3_attn_scores(
 // p_t = bf16(exp(s_t - max) * (1 / sum)) and, for each of its 16 dims, the
 // 16 residue-class FMA chains over ascending t (one chain per chunk, chunks
 // added in order), combined by the fixed class tree ((c0 + c1) + (c2 + c3))
-// ... as attention_tail does. The exponentials of a chunk are computed once
-// by all threads into LDS; the block's 32-byte slice of the V rows goes
-// through registers into LDS in 1024-row tiles, each tile loaded while the
-// previous one's chains run; the chains take their operands 16 steps at a
-// time from LDS. spitch: a multiple of 512.
-extern "C" __global__ __launch_bounds__(256) void xpu_q3_attn_pv(
+// ... as attention_tail does. spitch: a multiple of 512.
+//
+// Bound: latency (loads, exponentials, sum, chains one behind the other), so
+// each phase is short: a thread takes the exponentials of eight consecutive
+// positions (a canonical lane's slots) and keeps them in registers, every
+// wavefront sums the chunk itself from one LDS copy, and the probabilities
+// lie class by class in LDS (four steps per read). Waves 0 and 1 run the
+// chains of 8 dims each (thread: one class, two dims) on V loads of 16 bytes
+// per lane, 64 positions at a time, whose lanes exchange dwords (four swaps)
+// instead of a pass through LDS; 2048 positions are in flight, half of them
+// out before the softmax. Cycles of a wavefront (median, 0.6B, 2048
+// positions): 21.7K with V tiles through LDS and the denominator on one
+// wavefront, 18.8K with 2-byte loads of one dim per thread (8.2 us a launch),
+// 12.3K here (7.1 us).
+extern "C" __global__ __launch_bounds__(256, 1) void xpu_q3_attn_pv(
     const float *__restrict__ scores, const float *__restrict__ maxima, const uint16_t *__restrict__ vcache,
     uint16_t *__restrict__ out, const uint32_t *__restrict__ state, uint32_t heads, uint32_t kv_heads,
     uint32_t max_seq, uint32_t spitch, uint32_t parts) {
   XPU_STAMP(xpu::kStampQ3Pv);
-  constexpr uint32_t kDims = 16, kChunk = xpu::kAttnChunk, kTile = 1024, kRows = kTile / 128, kMaxChunks = 64;
-  constexpr uint32_t kPer = kChunk / 256, kBatch = 16;
-  extern __shared__ __align__(16) uint8_t pv_lds[];
-  float *pbuf = reinterpret_cast<float *>(pv_lds);                           // kChunk floats
-  uint16_t *vt = reinterpret_cast<uint16_t *>(pv_lds + kChunk * 4);         // kChunk x 16 codes
-  float *csum = reinterpret_cast<float *>(pv_lds + kChunk * 4 + kChunk * kDims * 2);
-  float *wsum = csum + kMaxChunks;                                           // 4 x 16
+  constexpr uint32_t kChunk = xpu::kAttnChunk, kBatch = 8, kRing = 4;  // V loads per batch, batches in flight
+  constexpr uint32_t kSpan = 64 * kBatch;                              // positions per batch
+  // a class's probabilities: the pitch puts the writes of classes c and c + 8
+  // and the 16-byte reads of the 16 classes on distinct banks
+  constexpr uint32_t kPitch = kChunk / 16 + 4;
+  static_assert(kChunk % (kRing * kSpan) == 0 && kChunk == 8 * 512, "whole rings per chunk; two 512-position rows per wave");
+  __shared__ __align__(16) float ebuf[kChunk];       // exponentials by position
+  __shared__ __align__(16) float pbuf[16 * kPitch];  // probabilities by class, then position / 16
   uint32_t kv, head, g;
   split_block(blockIdx.x, heads, kv_heads, kv, head, g);
   const uint32_t tid = threadIdx.x, lane = xpu::lane_id();
@@ -944,128 +956,156 @@ extern "C" __global__ __launch_bounds__(256) void xpu_q3_attn_pv(
   if (pos >= max_seq) return;
   const uint32_t n = pos + 1, nchunks = (n + kChunk - 1) / kChunk;
   const float *srow = scores + static_cast<uint64_t>(head) * spitch;
-  // the chunk's scores (16 per thread, positions tid + 256 k, index clamped)
-  auto load_s = [&](uint32_t base, uint32_t len, float (&sv)[kPer]) {
+  // this thread's scores of a chunk: positions 512 j + 8 lane + e, j = wave, wave + 4 (rows past the context
+  // repeat its last row)
+  auto load_s = [&](uint32_t base, float4 (&sv)[4]) {
 #pragma unroll
-    for (int k = 0; k < static_cast<int>(kPer); ++k) sv[k] = srow[base + min(tid + 256u * k, len - 1)];
+    for (uint32_t q = 0; q < 2; ++q) {
+      const float4 *p = reinterpret_cast<const float4 *>(
+          srow + min(base / 512u + wave + 4u * q, (n - 1u) / 512u) * 512u + lane * 8u);
+      sv[2 * q] = p[0];
+      sv[2 * q + 1] = p[1];
+    }
   };
-  // V rows from the chunk-major cache (dims 16 g .. 16 g + 15 are cache
-  // chunks 2 g and 2 g + 1): waves 0, 1 read chunk 2 g and waves 2, 3 chunk
-  // 2 g + 1, lane l of wave w rows 128 k + 64 (w % 2) + l of a tile, so a
-  // load instruction reads 1 KiB contiguous. The loads go through a buffer
-  // descriptor that ends at the context: rows past it read zeros without a
-  // memory access, and no load is behind a branch (which would make the
-  // compiler wait for all earlier loads before each one).
-  const uint32_t vr = (wave & 1u) * 64u + lane, vh = (wave >> 1) * 8u;
+  // V of cache chunk 2 g + wave (dims 8 (2 g + wave) .. + 7) for waves 0 and 1:
+  // lane l of load u takes position 64 u + l of the batch (class l % 16), through
+  // a descriptor that ends at the context (rows past it read zeros without a
+  // memory access; waves 2 and 3 read none)
+  const bool chains = wave < 2;
   const uint16_t *vb = vcache + static_cast<uint64_t>(kv) * max_seq * xpu::kHeadDim +
-                       static_cast<uint64_t>(2u * g + (wave >> 1)) * max_seq * 8u;
-  const __amdgpu_buffer_rsrc_t vrs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(vb), static_cast<short>(0), static_cast<int>(n * 16u),
-                                        0x00020000);
-  auto load_tile = [&](uint32_t t0, u32x4 (&vv)[kRows]) {  // rows t0 .. t0 + 1023 of the context
+                       static_cast<uint64_t>(2u * g + (wave & 1u)) * max_seq * 8u;
+  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t *>(vb), static_cast<short>(0), chains ? static_cast<int>(n * 16u) : 0, 0x00020000);
+  u32x4 vv[kRing][kBatch];
+  auto load_v = [&](uint32_t batch, u32x4 (&v)[kBatch]) {
 #pragma unroll
-    for (int k = 0; k < static_cast<int>(kRows); ++k)
-      vv[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vrs, (t0 + k * 128u + vr) * 16u, 0, 0));
+    for (uint32_t u = 0; u < kBatch; ++u)
+      v[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                           vrs, lane * 16u + (u % 4u) * 1024u, batch * (kSpan * 16u) + u / 4u * 4096u, 0));
   };
-  auto store_tile = [&](uint32_t r0, const u32x4 (&vv)[kRows]) {  // into chunk rows r0 .. r0 + 1023
+  float4 sv[4];
+  load_s(0, sv);
 #pragma unroll
-    for (int k = 0; k < static_cast<int>(kRows); ++k)
-      *reinterpret_cast<u32x4 *>(vt + (r0 + k * 128u + vr) * kDims + vh) = vv[k];
-  };
-  float sv[kPer];
-  u32x4 vv[kRows];
-  load_s(0, min(kChunk, n), sv);
-  load_tile(0, vv);
+  for (uint32_t k = 0; k < kRing / 2; ++k) load_v(k, vv[k]);
   const float mx = xpu::wave_reduce(pm, [](float x, float y) { return fmaxf(x, y); });
   XPU_PHASE(0);  // (stamps build) the softmax maximum
-  auto exps = [&](uint32_t len, const float (&s)[kPer], bool scaled, float sinv) {
+  float ex[16];  // exponentials of this thread's positions, 0 past the context
+  auto exps = [&](uint32_t base, const float4 (&s)[4]) {
 #pragma unroll
-    for (int k = 0; k < static_cast<int>(kPer); ++k) {
-      const uint32_t i = tid + 256u * k;
-      if (i < len) {
-        const float e = xpu::canonical_exp(s[k] - mx);
-        pbuf[i] = scaled ? xpu::round_bf16(e * sinv) : e;
+    for (uint32_t i = 0; i < 4; ++i) {
+      const float x[4] = {s[i].x, s[i].y, s[i].z, s[i].w};
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) {
+        const uint32_t t = base + (wave + 4u * (i >> 1)) * 512u + lane * 8u + 4u * (i & 1u) + e;
+        ex[4 * i + e] = t < n ? xpu::canonical_exp_nonpos(x[e] - mx) : 0.0f;
       }
     }
   };
+  float total = 0.0f;
   for (uint32_t c = 0; c < nchunks; ++c) {
-    const uint32_t base = c * kChunk, len = min(kChunk, n - base);
+    const uint32_t base = c * kChunk, rows = (min(kChunk, n - base) + 511u) / 512u;
     if (c) {
-      float sc[kPer];
-      load_s(base, len, sc);
-      exps(len, sc, false, 0.0f);
+      float4 sc[4];
+      load_s(base, sc);
+      __syncthreads();  // the previous chunk's exponentials are no longer read
+      exps(base, sc);
     } else {
-      exps(len, sv, false, 0.0f);
+      exps(base, sv);
     }
-    __syncthreads();
-    if (wave == 0) {
-      float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      for (uint32_t j = 0; j < len; j += 512u) {
-        const float4 a = *reinterpret_cast<const float4 *>(pbuf + j + lane * 8u);
-        const float4 b = *reinterpret_cast<const float4 *>(pbuf + j + lane * 8u + 4u);
-        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (j + lane * 8u + e < len) acc[e] = acc[e] + x[e];
-      }
-      const float cs = xpu::wave_butterfly(xpu::fold8(acc));
-      if (lane == 0) csum[c] = cs;
+    for (uint32_t i = 0; i < 4; ++i)
+      *reinterpret_cast<float4 *>(ebuf + (wave + 4u * (i >> 1)) * 512u + lane * 8u + 4u * (i & 1u)) =
+          float4{ex[4 * i], ex[4 * i + 1], ex[4 * i + 2], ex[4 * i + 3]};
+    if (c == 0) {  // (all of them ahead of the exponentials delay the scores)
+#pragma unroll
+      for (uint32_t k = kRing / 2; k < kRing; ++k) load_v(k, vv[k]);
     }
     __syncthreads();
+    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (uint32_t j = 0; j < rows; ++j) {
+      const float4 a = *reinterpret_cast<const float4 *>(ebuf + j * 512u + lane * 8u);
+      const float4 b = *reinterpret_cast<const float4 *>(ebuf + j * 512u + lane * 8u + 4u);
+      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = acc[e] + x[e];  // past the context: + 0, which leaves a sum from +0 as it is
+    }
+    total = total + xpu::wave_butterfly(xpu::fold8(acc));
   }
   XPU_PHASE(1);  // (stamps build) exponentials and the denominator's chunk sums
-  float total = 0.0f;
-  for (uint32_t c = 0; c < nchunks; ++c) total = total + csum[c];
   const float inv = 1.0f / total;
-  // P.V: lane l of wave w owns residue class 4 w + l / 16 and dim l % 16
-  const uint32_t cls = wave * 4u + (lane >> 4), d = lane & 15u;
-  float tot = 0.0f;
+  const uint32_t cls = lane & 15u, pair = lane >> 4;  // of the chains: dims 2 pair, 2 pair + 1 of the wave's 8
+  float tot[2] = {0.0f, 0.0f};
   for (uint32_t c = 0; c < nchunks; ++c) {
-    const uint32_t base = c * kChunk, len = min(kChunk, n - base);
-    if (c) {
-      __syncthreads();  // the previous chunk's probabilities and rows are no longer read
-      float sc[kPer];
-      load_s(base, len, sc);
-      exps(len, sc, true, inv);
-    } else if (nchunks == 1) {
-      for (uint32_t i = tid; i < len; i += 256u) pbuf[i] = xpu::round_bf16(pbuf[i] * inv);
-    } else {
-      exps(len, sv, true, inv);
+    const uint32_t base = c * kChunk;
+    if (nchunks > 1) {
+      if (c) __syncthreads();  // the previous chunk's probabilities are no longer read
+      float4 sc[4];
+      load_s(base, sc);
+      exps(base, sc);
     }
+    // position 512 j + 8 L + e: class 8 (L % 2) + e, step 32 j + L / 2
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i)
+      pbuf[((lane & 1u) * 8u + (i & 7u)) * kPitch + (wave + 4u * (i >> 3)) * 32u + (lane >> 1)] =
+          xpu::round_bf16(ex[i] * inv);
+    __syncthreads();
     XPU_PHASE(2);  // (stamps build) the (last) chunk's probabilities
-    float part = 0.0f;
-    for (uint32_t i0 = 0; i0 < len; i0 += kTile) {
-      store_tile(i0, vv);  // a region of the chunk's rows that no chain reads yet
-      load_tile(base + i0 + kTile, vv);  // the next tile (zeros past the context)
-      __syncthreads();  // the tile (and the chunk's probabilities) in LDS
-      // rows i0 + cls, i0 + cls + 16, ... of the tile, 16 at a time: the
-      // operands of a batch are read before its FMAs
-      const uint32_t tend = min(i0 + kTile, len);
-      uint32_t t0 = i0 + cls;
-      for (; t0 + 16u * (kBatch - 1) < tend; t0 += 16u * kBatch) {
-        float pp[kBatch];
-        uint32_t v[kBatch];
+    if (!chains) continue;
+    float part[2] = {0.0f, 0.0f};
+    const float *prow = pbuf + cls * kPitch;
+    // the steps of one batch; WHOLE: all inside the context
+    auto chain = [&](auto whole, const u32x4 (&vb8)[kBatch], uint32_t b, uint32_t t0) {
 #pragma unroll
-        for (int u = 0; u < static_cast<int>(kBatch); ++u) {
-          pp[u] = pbuf[t0 + 16u * u];
-          v[u] = vt[(t0 + 16u * u) * kDims + d];
+      for (uint32_t u = 0; u < kBatch; ++u) {
+        // lane (class, r) has dims 0 .. 7 of step 4 u + r: the 4 x 4 exchange
+        // over the lanes of a class leaves it dim pair r of steps 4 u .. 4 u + 3
+        const auto s02 = __builtin_amdgcn_permlane32_swap(vb8[u].x, vb8[u].z, false, false);
+        const auto s13 = __builtin_amdgcn_permlane32_swap(vb8[u].y, vb8[u].w, false, false);
+        const auto s01 = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+        const auto s23 = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+        const uint32_t v[4] = {s01[0], s01[1], s23[0], s23[1]};
+        const float4 p4 = *reinterpret_cast<const float4 *>(prow + b * (kSpan / 16u) + 4u * u);
+        const float pp[4] = {p4.x, p4.y, p4.z, p4.w};
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) {
+          const float lo = __builtin_fmaf(pp[w], xpu::lo16<xpu::kBf16>(v[w]), part[0]);
+          const float hi = __builtin_fmaf(pp[w], xpu::hi16<xpu::kBf16>(v[w]), part[1]);
+          const bool live = decltype(whole)::value || t0 + u * 64u + w * 16u + cls < n;
+          part[0] = live ? lo : part[0];
+          part[1] = live ? hi : part[1];
         }
-#pragma unroll
-        for (int u = 0; u < static_cast<int>(kBatch); ++u) part = __builtin_fmaf(pp[u], xpu::bf16_to_f32(v[u]), part);
       }
-      for (; t0 < tend; t0 += 16u) part = __builtin_fmaf(pbuf[t0], xpu::bf16_to_f32(vt[t0 * kDims + d]), part);
+    };
+    for (uint32_t b0 = 0; b0 < kChunk / kSpan; b0 += kRing) {
+      if (base + b0 * kSpan >= n) break;
+#pragma unroll
+      for (uint32_t k = 0; k < kRing; ++k) {
+        const uint32_t t0 = base + (b0 + k) * kSpan;
+        if (t0 + kSpan > n) {
+          if (t0 < n) chain(std::false_type{}, vv[k], b0 + k, t0);
+          break;
+        }
+        chain(std::true_type{}, vv[k], b0 + k, t0);
+        load_v(t0 / kSpan + kRing, vv[k]);
+      }
     }
-    tot = tot + part;
+    tot[0] = tot[0] + part[0];
+    tot[1] = tot[1] + part[1];
   }
-  XPU_PHASE(3);  // (stamps build) the V tiles and their chains
-  const float pair = tot + xpu::xor16_f(tot);  // (c0 + c1), (c2 + c3)
-  const float sum = pair + xpu::xor32_f(pair); // (c0 + c1) + (c2 + c3)
-  if (lane < 16) wsum[wave * kDims + lane] = sum;
-  __syncthreads();
-  if (tid < kDims) {
-    const float r = (wsum[tid] + wsum[kDims + tid]) + (wsum[2 * kDims + tid] + wsum[3 * kDims + tid]);
-    out[head * xpu::kHeadDim + g * kDims + tid] = static_cast<uint16_t>(xpu::f32_to_bf16(r));
+  XPU_PHASE(3);  // (stamps build) the chains
+  if (!chains) return;
+  uint32_t code[2];
+#pragma unroll
+  for (uint32_t e = 0; e < 2; ++e) {
+    float v = tot[e];
+    v = v + xpu::dpp_f<0xB1>(v);   // xor 1: c0 + c1
+    v = v + xpu::dpp_f<0x4E>(v);   // xor 2: (c0 + c1) + (c2 + c3)
+    v = v + xpu::dpp_f<0x141>(v);  // row_half_mirror: of eight classes
+    v = v + xpu::xor8_f(v);
+    code[e] = xpu::f32_to_bf16(v);
   }
+  if (cls == 0)
+    *reinterpret_cast<uint32_t *>(out + head * xpu::kHeadDim + (2u * g + wave) * 8u + 2u * pair) = code[0] | (code[1] << 16);
 }
 
 // Reduce the per-block argmax partials; token = 0xffffffff if any logit was

@@ -361,10 +361,8 @@ int setup_launches(xpu_qwen3 &e) {
   e.pv_l.k = e.rt->find_exact("xpu_q3_attn_pv");
   e.scores_l.grid = c.heads * e.att_parts;
   e.pv_l.grid = c.heads * 8;  // 16 output dims per block
-  // probabilities (4096 floats) + V rows (4096 x 16 codes) of a softmax
-  // chunk + 64 chunk sums + 4 x 16 wave partials
-  e.pv_l.shared = 4096 * 4 + 4096 * 16 * 2 + 64 * 4 + 64 * 4;
-  e.split_ok = e.scores_l.k && e.pv_l.k && e.max_seq <= 64u * 4096u && e.pv_l.shared <= e.rt->max_shared;
+  e.pv_l.shared = 0;
+  e.split_ok = e.scores_l.k && e.pv_l.k && e.max_seq <= 64u * 4096u;
   if ((rc = pick("xpu_q3_gemv_residual_r1", qd, "xpu_q3_gemv_residual_r1", e.o_l))) return rc;
   e.o_l.grid = std::min(cap_for(c.hidden, qd), (c.hidden + 3) / 4);
   if ((rc = pick("xpu_q3_norm_gemv_swiglu_r2", c.hidden, "xpu_q3_norm_gemv_swiglu_r2", e.gu_l))) return rc;

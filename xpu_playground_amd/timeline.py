@@ -49,7 +49,7 @@ PHASES = {
     "attention": ["operand loads, QK-norm, RoPE", "scores and their maximum",
                   "exponentials and lane sums", "denominator, P.V chains, combine, store"],
     "attn_pv": ["softmax maximum (score and V loads issued)", "exponentials and denominator",
-                "probabilities", "V tiles and their chains", "combine and store"],
+                "probabilities", "V chains", "combine and store"],
 }
 
 
