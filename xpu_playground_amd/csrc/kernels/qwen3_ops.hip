@@ -931,9 +931,9 @@ extern "C" __global__ __launch_bounds__(256) void xpu_q3_attn_scores(
 // per lane, 64 positions at a time, whose lanes exchange dwords (four swaps)
 // instead of a pass through LDS; 2048 positions are in flight, half of them
 // out before the softmax. Cycles of a wavefront (median, 0.6B, 2048
-// positions): 21.7K with V tiles through LDS and the denominator on one
-// wavefront, 18.8K with 2-byte loads of one dim per thread (8.2 us a launch),
-// 12.3K here (7.1 us).
+// positions): 21.7K (9.4 us a launch) with V tiles through LDS and the
+// denominator on one wavefront, 18.8K (8.2 us) with 2-byte loads of one dim
+// per thread, 12.3K here (7.1 us).
 extern "C" __global__ __launch_bounds__(256, 1) void xpu_q3_attn_pv(
     const float *__restrict__ scores, const float *__restrict__ maxima, const uint16_t *__restrict__ vcache,
     uint16_t *__restrict__ out, const uint32_t *__restrict__ state, uint32_t heads, uint32_t kv_heads,
