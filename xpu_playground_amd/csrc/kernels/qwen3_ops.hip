@@ -970,7 +970,8 @@ extern "C" __global__ __launch_bounds__(256, 1) void xpu_q3_attn_pv(
   // V of cache chunk 2 g + wave (dims 8 (2 g + wave) .. + 7) for waves 0 and 1:
   // lane l of load u takes position 64 u + l of the batch (class l % 16), through
   // a descriptor that ends at the context (rows past it read zeros without a
-  // memory access; waves 2 and 3 read none)
+  // memory access; waves 2 and 3 read none). The whole offset is in the vector
+  // operand: a buffer load's scalar offset is no part of its bounds check.
   const bool chains = wave < 2;
   const uint16_t *vb = vcache + static_cast<uint64_t>(kv) * max_seq * xpu::kHeadDim +
                        static_cast<uint64_t>(2u * g + (wave & 1u)) * max_seq * 8u;
@@ -981,7 +982,7 @@ extern "C" __global__ __launch_bounds__(256, 1) void xpu_q3_attn_pv(
 #pragma unroll
     for (uint32_t u = 0; u < kBatch; ++u)
       v[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                           vrs, lane * 16u + (u % 4u) * 1024u, batch * (kSpan * 16u) + u / 4u * 4096u, 0));
+                                           vrs, (batch * kSpan + u * 64u + lane) * 16u, 0, 0));
   };
   float4 sv[4];
   load_s(0, sv);
