@@ -1,5 +1,6 @@
 """Properties of the compiled kernels that no result shows, read from the code
-objects built from this source: which loads the hardware bounds-checks."""
+objects built from this source: which loads the hardware bounds-checks, and in
+which order loads that hide each other's latency go out."""
 import os
 import re
 import subprocess
@@ -28,3 +29,11 @@ def test_split_pv_loads_are_bounds_checked(code_object):
     for i in loads:
         m = re.fullmatch(r"buffer_load_dwordx4 v\[\d+:\d+\], v\d+, s\[\d+:\d+\], (\S+) offen( offset:\d+)?", i)
         assert m and m.group(1) == "0", i
+
+
+def test_split_pv_asks_for_the_scores_before_v():
+    """Loads return in order, so V rows asked for ahead of the scores would be
+    waited for before the first exponential."""
+    loads = [i.split()[0] for i in assembly("xpu_kernels.hsaco", "xpu_q3_attn_pv") if re.match(r"(global|buffer)_load", i)]
+    # the partial maximum, four score vectors, the first half of the V ring
+    assert loads[:21] == ["global_load_dword"] + ["global_load_dwordx4"] * 4 + ["buffer_load_dwordx4"] * 16

@@ -930,10 +930,12 @@ extern "C" __global__ __launch_bounds__(256) void xpu_q3_attn_scores(
 // chains of 8 dims each (thread: one class, two dims) on V loads of 16 bytes
 // per lane, 64 positions at a time, whose lanes exchange dwords (four swaps)
 // instead of a pass through LDS; 2048 positions are in flight, half of them
-// out before the softmax. Cycles of a wavefront (median, 0.6B, 2048
-// positions): 21.7K (9.4 us a launch) with V tiles through LDS and the
-// denominator on one wavefront, 18.8K (8.2 us) with 2-byte loads of one dim
-// per thread, 12.3K here (7.1 us).
+// out before the softmax and behind the loads of the scores, which the
+// exponentials would otherwise wait for together with V (2100 positions, kernel
+// trace: 7.9 us a launch against 8.1 with V first). Cycles of a wavefront
+// (median, 0.6B, 2048 positions, stamps build): 21.7K (9.4 us a launch) with V
+// tiles through LDS and the denominator on one wavefront, 18.8K (8.2 us) with
+// 2-byte loads of one dim per thread, 12.2K here (7.0 us).
 extern "C" __global__ __launch_bounds__(256, 1) void xpu_q3_attn_pv(
     const float *__restrict__ scores, const float *__restrict__ maxima, const uint16_t *__restrict__ vcache,
     uint16_t *__restrict__ out, const uint32_t *__restrict__ state, uint32_t heads, uint32_t kv_heads,
@@ -986,8 +988,12 @@ extern "C" __global__ __launch_bounds__(256, 1) void xpu_q3_attn_pv(
   };
   float4 sv[4];
   load_s(0, sv);
+  __builtin_amdgcn_sched_barrier(0);  // the scores go out first: waiting for them leaves V in flight
 #pragma unroll
   for (uint32_t k = 0; k < kRing / 2; ++k) load_v(k, vv[k]);
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i)  // (used in the loop, where the compiler would put their loads)
+    asm volatile("" : "+v"(sv[i].x), "+v"(sv[i].y), "+v"(sv[i].z), "+v"(sv[i].w));
   const float mx = xpu::wave_reduce(pm, [](float x, float y) { return fmaxf(x, y); });
   XPU_PHASE(0);  // (stamps build) the softmax maximum
   float ex[16];  // exponentials of this thread's positions, 0 past the context
