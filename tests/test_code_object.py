@@ -1,6 +1,7 @@
 """Properties of the compiled kernels that no result shows, read from the code
-objects built from this source: which loads the hardware bounds-checks, and in
-which order loads that hide each other's latency go out."""
+objects built from this source: which loads the hardware bounds-checks, in which
+order loads that hide each other's latency go out, and how many wavefronts
+the registers leave room for."""
 import os
 import re
 import subprocess
@@ -37,3 +38,20 @@ def test_split_pv_asks_for_the_scores_before_v():
     loads = [i.split()[0] for i in assembly("xpu_kernels.hsaco", "xpu_q3_attn_pv") if re.match(r"(global|buffer)_load", i)]
     # the partial maximum, four score vectors, the first half of the V ring
     assert loads[:21] == ["global_load_dword"] + ["global_load_dwordx4"] * 4 + ["buffer_load_dwordx4"] * 16
+
+
+def vgprs(kernel):
+    notes = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes",
+                            os.path.join(xpu.BUILD_DIR, "xpu_kernels.hsaco")],
+                           capture_output=True, text=True, check=True).stdout
+    block = next(b for b in notes.split("  - .agpr_count:")[1:] if re.search(rf"\.symbol:\s+{kernel}\.kd", b))
+    return int(re.search(r"\.vgpr_count:\s+(\d+)", block).group(1))
+
+
+@pytest.mark.parametrize("kernel,waves", [
+    ("xpu_q3_norm_gemv_r2", 4), ("xpu_q3_norm_gemv_swiglu_r2", 4), ("xpu_q3_norm_gemv_logits_r2", 4),
+    ("xpu_q3_gemv_residual_r1", 6)])
+def test_staged_decode_kernels_keep_their_wavefronts(kernel, waves):
+    """Wavefronts per SIMD that 512 registers in steps of 8 allow the decode
+    kernels of wide models, which stream their weights on that many."""
+    assert 512 // ((vgprs(kernel) + 7) // 8 * 8) >= waves

@@ -33,7 +33,13 @@ XPU_DEVICE void gemv_entry(const uint16_t *__restrict__ A, const uint16_t *__res
     const uint32_t row0 = base + wave * R;
     if (row0 >= M) continue;
     float out[R];
-    gemv_rows<DT, R, U, VEC>(A, lda, K, M, xs, row0, out);
+    // Row ends ahead of the batches for short rows (two-chunk batches); for
+    // long ones the loads ahead of the first batch cost 16384^2 fp16 5%. The
+    // decode kernels load them where they are used: their widths mostly have
+    // no such end, and its registers would cost them a wavefront per SIMD
+    // (135 registers instead of 123; no difference in time was measured at
+    // hidden 5120, 322 us a token for two layers either way).
+    gemv_rows<DT, R, U, VEC, U == 2>(A, lda, K, M, xs, row0, out);
     const uint32_t lane = lane_id();
 #pragma unroll
     for (int r = 0; r < R; ++r)

@@ -128,8 +128,10 @@ XPU_DEVICE void gemv_load_batch(u32x4 (&buf)[U][R], const uint16_t *const (&rows
 // vector xs. All lanes must be active. When use_first is set (wave-uniform),
 // `first` holds the rows' first batch (chunks 0..U-1), loaded earlier by the
 // caller with gemv_load_batch so that its latency overlaps other work; it is
-// only used when K has at least U full chunks.
-template <int DT, int R, int U, bool VEC, bool PAIRED = false>
+// only used when K has at least U full chunks. EARLY: the chunk that crosses K
+// and, for U = 2, the full chunk left over after the batches are loaded ahead
+// of them, so that a row does not wait for its end on its own.
+template <int DT, int R, int U, bool VEC, bool PAIRED = false, bool EARLY = false>
 XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, uint32_t K,
                                 uint32_t M, const uint16_t *xs, uint32_t row0, float (&out)[R],
                                 uint32_t pair_offset, const u32x4 (&first)[U][R], bool use_first) {
@@ -153,21 +155,17 @@ XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, ui
     for (int u = 0; u < U; ++u)
       fma_chunk<DT, R>(acc, buf[u], *reinterpret_cast<const u32x4 *>(xl + (j0 + u) * 512u));
   };
-  // With two-chunk batches (short rows) the chunk that crosses K and the full
-  // chunk left over after the batches are loaded ahead of them, so that a row
-  // does not wait for its end on its own. Long rows load them where they are
-  // used: the loads ahead of the first batch cost 16384^2 fp16 5%. A row of
-  // fewer than 8 columns has no 8 codes to load.
-  constexpr bool kEarly = U == 2;
+  // a row of fewer than 8 columns has no 8 codes to load
+  static_assert(!EARLY || U == 2, "one chunk is left over after the batches");
   const uint32_t tail_col = nfull * 512u + lane * 8u;
-  const bool tail8 = K % 512u != 0 && K >= 8u, spare = kEarly && nfull % 2u != 0;
+  const bool tail8 = K % 512u != 0 && K >= 8u, spare = EARLY && nfull % 2u != 0;
   u32x4 tail[R], over[R];
   auto load_tail = [&]() {
     const uint32_t at = tail_col < K - 8u ? tail_col : K - 8u;
 #pragma unroll
     for (int r = 0; r < R; ++r) tail[r] = load_row8<VEC>(rows[r] + static_cast<int32_t>(at - lane * 8u));
   };
-  if (kEarly && tail8) load_tail();
+  if (EARLY && tail8) load_tail();
   if (spare) {
 #pragma unroll
     for (int r = 0; r < R; ++r) over[r] = load_row8<VEC>(rows[r] + (nfull - 1u) * 512u);
@@ -200,14 +198,14 @@ XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, ui
     fma_chunk<DT, R>(acc, over, *reinterpret_cast<const u32x4 *>(xl + j * 512u));
     ++j;
   }
-  if constexpr (!kEarly)
+  if constexpr (!EARLY)
     for (; j < nfull; ++j) {
       u32x4 a[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) a[r] = load_row8<VEC>(rows[r] + j * 512u);
       fma_chunk<DT, R>(acc, a, *reinterpret_cast<const u32x4 *>(xl + j * 512u));
     }
-  if constexpr (VEC && !kEarly) {
+  if constexpr (VEC && !EARLY) {
     if (K % 512u && tail_col < K) {
       u32x4 a[R];
 #pragma unroll
@@ -217,7 +215,7 @@ XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, ui
   } else if (K % 512u) {
     u32x4 a[R];
     if (tail8) {
-      if (!kEarly) load_tail();
+      if (!EARLY) load_tail();
 #pragma unroll
       for (int r = 0; r < R; ++r) a[r] = VEC ? tail[r] : cut_tail(tail[r], tail_col, K);
     } else {
@@ -235,11 +233,11 @@ XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, ui
   for (int r = 0; r < R; ++r) out[r] = wave_butterfly(fold8(acc[r]));
 }
 
-template <int DT, int R, int U, bool VEC, bool PAIRED = false>
+template <int DT, int R, int U, bool VEC, bool EARLY = false>
 XPU_DEVICE void gemv_rows(const uint16_t *__restrict__ A, uint64_t lda, uint32_t K, uint32_t M,
-                          const uint16_t *xs, uint32_t row0, float (&out)[R], uint32_t pair_offset = 0) {
+                          const uint16_t *xs, uint32_t row0, float (&out)[R]) {
   u32x4 unused[U][R];
-  gemv_rows_first<DT, R, U, VEC, PAIRED>(A, lda, K, M, xs, row0, out, pair_offset, unused, false);
+  gemv_rows_first<DT, R, U, VEC, false, EARLY>(A, lda, K, M, xs, row0, out, 0, unused, false);
 }
 
 }  // namespace xpu
