@@ -912,8 +912,8 @@ XPU_GEMM_DMA_VARIANT(xpu_gemm_fp16_t128_dma, xpu::kFp16, 2, 2, 64, 2, 2, 2, 2, t
 XPU_GEMM_DMA_VARIANT(xpu_gemm_bf16_t128_dmau, xpu::kBf16, 2, 2, 64, 2, 2, 2, 2, false, false)
 XPU_GEMM_DMA_VARIANT(xpu_gemm_fp16_t128_dmau, xpu::kFp16, 2, 2, 64, 2, 2, 2, 2, false, false)
 
-// Split K for [k][n] products that leave most compute units idle even with
-// small tiles (a small output with a long reduction): FP32 partials of
+// Split K for [k][n] products that leave most compute units idle with whole
+// chains (a small output with a long reduction): FP32 partials of
 // each K range (kb slices, a multiple of the stages), added by
 // xpu_gemm_splitk_reduce_any; _edge as for the whole-K kernels.
 #define XPU_GEMM_PART_KN(NAME, DT, MI, NJ, S, P, MINB, EDGE, WN)                                           \
@@ -924,6 +924,10 @@ XPU_GEMM_DMA_VARIANT(xpu_gemm_fp16_t128_dmau, xpu::kFp16, 2, 2, 64, 2, 2, 2, 2, 
     xpu::dma::body<DT, MI, NJ, 64, S, P, 2, true, false, false, false, true, EDGE, WN>(A, B, C, M, N, K, kb, \
                                                                                       ldc, n_out);         \
   }
+XPU_GEMM_PART_KN(xpu_gemm_bf16_t128_part_dma, xpu::kBf16, 2, 2, 2, 2, 2, false, 2)
+XPU_GEMM_PART_KN(xpu_gemm_bf16_t128_part_dma_edge, xpu::kBf16, 2, 2, 2, 2, 2, true, 2)
+XPU_GEMM_PART_KN(xpu_gemm_fp16_t128_part_dma, xpu::kFp16, 2, 2, 2, 2, 2, false, 2)
+XPU_GEMM_PART_KN(xpu_gemm_fp16_t128_part_dma_edge, xpu::kFp16, 2, 2, 2, 2, 2, true, 2)
 
 // Small tiles for outputs that leave compute units idle or half loaded at
 // 128 x 128: 32 x 128 (1 x 4 wavefronts of 32 x 32, four stages of 20 KiB)
