@@ -55,3 +55,9 @@ def test_staged_decode_kernels_keep_their_wavefronts(kernel, waves):
     """Wavefronts per SIMD that 512 registers in steps of 8 allow the decode
     kernels of wide models, which stream their weights on that many."""
     assert 512 // ((vgprs(kernel) + 7) // 8 * 8) >= waves
+
+
+def test_whole_batch_gemv_keeps_no_row_ends():
+    """Rows of whole batches do not pay for ends loaded ahead (107 registers
+    without them, 119 with)."""
+    assert vgprs("xpu_gemv_bf16_r2u2_vec") < vgprs("xpu_gemv_bf16_r2u2_ends")

@@ -64,7 +64,7 @@ def test_gemv_matches_oracle(rt, dtype, m, k, lda):
 @pytest.mark.parametrize("m,k,lda", [(64, 512, 512), (37, 1000, 1000), (1000, 1032, 1040), (5, 3, 7)])
 def test_gemv_pointers_two_bytes_past_alignment(rt, dtype, m, k, lda):
     # A, x and y start 2 bytes past a 16-byte boundary, which the 16-byte
-    # loads of the vector variants cannot take: the 16-bit-load variant runs.
+    # loads of the vector variants cannot take: the unaligned variant runs.
     # Guard codes around y catch any store outside it.
     print(f"gemv unaligned pointers dtype={dtype} m={m} k={k} lda={lda}", flush=True)
     a = orc.uniform(m * lda, 300 + m, dtype)

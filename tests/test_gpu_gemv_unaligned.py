@@ -40,3 +40,12 @@ def test_unaligned_rows(rt, dtype, m, k, pad, offset):
             rt.free(p)
     assert np.array_equal(y[:m], want)
     assert np.all(y[m:] == 0x7FC1)
+
+
+@pytest.mark.parametrize("dtype", [xpu.BF16, xpu.FP16])
+@pytest.mark.parametrize("k", [8, 504, 1024, 1032, 2048, 3072, 4088, 4096, 4104, 5120, 7168, 7680, 8184, 8192, 8200])
+@pytest.mark.parametrize("m", [1, 9])
+def test_aligned_rows_with_and_without_ends(rt, dtype, m, k):
+    """Aligned rows around the change of kernels: row ends loaded ahead of the
+    batches, except where 4096 columns or more are whole batches."""
+    test_unaligned_rows(rt, dtype, m, k, 8, 8)

@@ -49,11 +49,13 @@ int plan_gemv(const xpu_runtime &rt, int dtype, const void *A, const void *x, ui
   // instead: 151936 x 1024 86.5 -> 52.8 us, 20000 x 1024 12.7 -> 8.4,
   // 16384 x 500 10.0 -> 5.2, 12000 x 10000 58.5 -> 38.9.
   const uint64_t tiles = (static_cast<uint64_t>(M) + 4 * rows - 1) / (4 * rows);
+  const bool whole = K >= 4096 && K % (short_rows ? 1024 : 2048) == 0;
   const uint32_t per_cu =
       K >= 4096 && K % 2048 == 0 ? 1u : plan.shared ? std::min(4u, std::max(1u, rt.max_shared / plan.shared)) : 1u;
   plan.grid = static_cast<uint32_t>(std::min<uint64_t>(tiles, uint64_t{rt.compute_units} * per_cu));
   plan.kernel = std::string("xpu_gemv_") + (dtype ? "fp16" : "bf16") + "_r" + std::to_string(rows) + "u" +
-                std::to_string(unroll) + (vec ? (global_x ? "_vecg" : "_vec") : "_any");
+                std::to_string(unroll) +
+                (!vec ? "_any" : global_x ? "_vecg" : short_rows && !whole ? "_ends" : "_vec");
   return XPU_OK;
 }
 

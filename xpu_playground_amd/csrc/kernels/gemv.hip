@@ -5,17 +5,17 @@
 // Launch: 256 threads (4 wavefronts, fixed at compile time); dynamic LDS = round_up(K, 512) * 2
 // bytes for the staged vector; the grid walks tiles of 4*R rows with a
 // grid-stride loop so each block stages the vector once. Any M, K >= 1 and
-// any leading dimension lda >= K are accepted; the _vec variants need A, x
-// 16-byte aligned and K, lda multiples of 8 (the host checks), the _any
-// variants load 16 bytes at any element. The _vecg variants read the vector from global memory
-// when it does not fit in LDS.
+// any leading dimension lda >= K are accepted; the _vec, _vecg and _ends
+// variants need A, x 16-byte aligned and K, lda multiples of 8 (the host
+// checks), the _any variants load 16 bytes at any element. The _vecg variants
+// read the vector from global memory when it does not fit in LDS.
 #include "gemv_core.hpp"
 
 namespace xpu {
 
 // XG: read the vector from global memory (cached loads) instead of LDS, for
 // vectors longer than the LDS holds; needs the _vec alignment conditions.
-template <int DT, int R, int U, bool VEC, bool XG = false>
+template <int DT, int R, int U, bool VEC, bool XG, bool EARLY>
 XPU_DEVICE void gemv_entry(const uint16_t *__restrict__ A, const uint16_t *__restrict__ x,
                            uint16_t *__restrict__ y, uint32_t M, uint32_t K, uint64_t lda) {
   extern __shared__ __align__(16) uint16_t lds_x[];
@@ -33,13 +33,7 @@ XPU_DEVICE void gemv_entry(const uint16_t *__restrict__ A, const uint16_t *__res
     const uint32_t row0 = base + wave * R;
     if (row0 >= M) continue;
     float out[R];
-    // Row ends ahead of the batches for short rows (two-chunk batches); for
-    // long ones the loads ahead of the first batch cost 16384^2 fp16 5%. The
-    // decode kernels load them where they are used: their widths mostly have
-    // no such end, and its registers would cost them a wavefront per SIMD
-    // (135 registers instead of 123; no difference in time was measured at
-    // hidden 5120, 322 us a token for two layers either way).
-    gemv_rows<DT, R, U, VEC, U == 2>(A, lda, K, M, xs, row0, out);
+    gemv_rows<DT, R, U, VEC, EARLY>(A, lda, K, M, xs, row0, out);
     const uint32_t lane = lane_id();
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -50,23 +44,30 @@ XPU_DEVICE void gemv_entry(const uint16_t *__restrict__ A, const uint16_t *__res
 
 }  // namespace xpu
 
-#define XPU_GEMV_VARIANT(NAME, DT, R, U, VEC, XG)                                          \
+#define XPU_GEMV_VARIANT(NAME, DT, R, U, VEC, XG, EARLY)                                   \
   extern "C" __global__ __launch_bounds__(256) void NAME(                                  \
       const uint16_t *__restrict__ A, const uint16_t *__restrict__ x,                      \
       uint16_t *__restrict__ y, uint32_t M, uint32_t K, uint64_t lda) {                    \
     XPU_STAMP(xpu::kStampGemv);                                                            \
-    xpu::gemv_entry<DT, R, U, VEC, XG>(A, x, y, M, K, lda);                                \
+    xpu::gemv_entry<DT, R, U, VEC, XG, EARLY>(A, x, y, M, K, lda);                         \
   }
+#define XPU_GEMV_TYPES(FORM, R, U, VEC, XG, EARLY)                                  \
+  XPU_GEMV_VARIANT(xpu_gemv_bf16_##FORM, xpu::kBf16, R, U, VEC, XG, EARLY)          \
+  XPU_GEMV_VARIANT(xpu_gemv_fp16_##FORM, xpu::kFp16, R, U, VEC, XG, EARLY)
 
-// name: xpu_gemv_<type>_r<R>u<U>_<vec|any|vecg>; R rows per wavefront, U
-// 512-column chunks per pipelined load batch
-#define XPU_GEMV_TYPES(R, U)                                                         \
-  XPU_GEMV_VARIANT(xpu_gemv_bf16_r##R##u##U##_vec, xpu::kBf16, R, U, true, false)   \
-  XPU_GEMV_VARIANT(xpu_gemv_fp16_r##R##u##U##_vec, xpu::kFp16, R, U, true, false)   \
-  XPU_GEMV_VARIANT(xpu_gemv_bf16_r##R##u##U##_any, xpu::kBf16, R, U, false, false)  \
-  XPU_GEMV_VARIANT(xpu_gemv_fp16_r##R##u##U##_any, xpu::kFp16, R, U, false, false)
-
-XPU_GEMV_TYPES(1, 4)
-XPU_GEMV_TYPES(2, 2)
-XPU_GEMV_VARIANT(xpu_gemv_bf16_r1u8_vecg, xpu::kBf16, 1, 8, true, true)
-XPU_GEMV_VARIANT(xpu_gemv_fp16_r1u8_vecg, xpu::kFp16, 1, 8, true, true)
+// name: xpu_gemv_<type>_r<R>u<U>_<vec|ends|any|vecg>; R rows per wavefront, U
+// 512-column chunks per pipelined load batch. The two-chunk forms _ends and
+// _any load the row's end (the chunk that crosses K, the full chunk left over)
+// ahead of the batches. Not where it costs: rows of 4096 columns or more that
+// are whole batches take _vec (65536 x 4096 76.2 us, 78.0 with _ends; x 8192
+// 151.5 and 155.8; x 1024 is the other way, 23.4 and 21.7), and so do long
+// rows (16384^2 fp16 5%) and the decode kernels, whose usual widths have no
+// such end and whose wavefronts per SIMD its registers would reduce (135
+// instead of 123; no difference in time was measured at hidden 5120, 322 us a
+// token for two layers either way).
+XPU_GEMV_TYPES(r1u4_vec, 1, 4, true, false, false)
+XPU_GEMV_TYPES(r1u4_any, 1, 4, false, false, false)
+XPU_GEMV_TYPES(r2u2_vec, 2, 2, true, false, false)
+XPU_GEMV_TYPES(r2u2_ends, 2, 2, true, false, true)
+XPU_GEMV_TYPES(r2u2_any, 2, 2, false, false, true)
+XPU_GEMV_TYPES(r1u8_vecg, 1, 8, true, true, false)
