@@ -49,3 +49,8 @@ def test_aligned_rows_with_and_without_ends(rt, dtype, m, k):
     """Aligned rows around the change of kernels: row ends loaded ahead of the
     batches, except where 4096 columns or more are whole batches."""
     test_unaligned_rows(rt, dtype, m, k, 8, 8)
+
+
+def test_many_rows_of_whole_batches(rt):
+    """More than 64 rows a compute unit: one block a unit instead of four."""
+    test_unaligned_rows(rt, xpu.BF16, 64 * rt.compute_units + 3, 5120, 0, 0)

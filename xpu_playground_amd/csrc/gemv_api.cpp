@@ -41,17 +41,21 @@ int plan_gemv(const xpu_runtime &rt, int dtype, const void *A, const void *x, ui
   const bool short_rows = !global_x && K <= 8192;
   const uint32_t rows = short_rows ? 2 : 1, unroll = global_x ? 8 : short_rows ? 2 : 4;
   plan.shared = global_x ? 0 : static_cast<uint32_t>(kpad * 2);
-  // grid-stride over 4-row tiles; each block stages the vector once. One
-  // block per compute unit where a row is whole load batches of 4096 columns
-  // or more (65536 x 4096 bf16 80.5 us against 82.5 with two to four,
-  // 32768 x 8192 81.9 against 82.5-83.7): its pipeline keeps the loads in
-  // flight. Up to four, as the LDS allows, where it drains at every row's end
-  // instead: 151936 x 1024 86.5 -> 52.8 us, 20000 x 1024 12.7 -> 8.4,
-  // 16384 x 500 10.0 -> 5.2, 12000 x 10000 58.5 -> 38.9.
+  // grid-stride over 4-row tiles; each block stages the vector once. One block
+  // per compute unit where a row of 4096 columns or more is whole load batches
+  // (1024 columns, long rows 2048; 65536 x 4096 bf16 76.2 us against 78.0-79.3
+  // with two to four, 32768 x 8192 79.4 against 79.3-81.1): its pipeline keeps
+  // the loads in flight. Up to four, as the LDS allows, where it drains at every
+  // row's end instead: 151936 x 1024 86.5 -> 52.8 us, 20000 x 1024 12.7 -> 8.4,
+  // 16384 x 500 10.0 -> 5.2, 12000 x 10000 58.5 -> 38.9; and for up to 64 rows a
+  // unit of K = 5120 or 7168 (16384 rows 27.4 -> 26.4 and 36.2 -> 36.0; 65536
+  // rows 95.0 against 96.9 and 129.5 against 134.5 with one and four).
   const uint64_t tiles = (static_cast<uint64_t>(M) + 4 * rows - 1) / (4 * rows);
   const bool whole = K >= 4096 && K % (short_rows ? 1024 : 2048) == 0;
   const uint32_t per_cu =
-      K >= 4096 && K % 2048 == 0 ? 1u : plan.shared ? std::min(4u, std::max(1u, rt.max_shared / plan.shared)) : 1u;
+      whole && (K % 2048 == 0 || M > 64 * rt.compute_units)
+          ? 1u
+          : plan.shared ? std::min(4u, std::max(1u, rt.max_shared / plan.shared)) : 1u;
   plan.grid = static_cast<uint32_t>(std::min<uint64_t>(tiles, uint64_t{rt.compute_units} * per_cu));
   plan.kernel = std::string("xpu_gemv_") + (dtype ? "fp16" : "bf16") + "_r" + std::to_string(rows) + "u" +
                 std::to_string(unroll) +
