@@ -195,7 +195,8 @@ int gemm_run(xpu_runtime *rt, int dtype, const void *A, const void *B, void *C, 
   const uint64_t split_bytes = static_cast<uint64_t>(M) * pitch * 4;
   const uint32_t limit = max_splits(rt->compute_units, tile, M, N, K);
   if (fixed_workspace && limit >= 2 && limit * split_bytes > fixed_capacity)
-    return set_error(XPU_ERR_INVALID, "xpu_gemm_noalloc: the split-K partials need " +
+    return set_error(XPU_ERR_INVALID, "xpu_gemm_noalloc: K may be split in up to " + std::to_string(limit) +
+                                          " ranges at this shape, whose partials would need " +
                                           std::to_string(limit * split_bytes) + " bytes, above the " +
                                           std::to_string(fixed_capacity) + "-byte scratch array");
   if (const SmallPlan plan = choose_small(rt->compute_units, tile, M, N, K, limit); plan.tile) {
