@@ -16,6 +16,7 @@ import pytest
 
 import oracle_lib as orc
 import xpu_playground_amd as xpu
+from test_gemm_plan import gemm_plan
 from test_gpu_gemm import check, gpu_gemm
 from xpu_playground_amd import Args
 
@@ -140,13 +141,15 @@ def test_ragged_baseline_shape_reads_operands_in_place(rt):
 
 @pytest.mark.parametrize("dtype", [xpu.BF16, xpu.FP16])
 @pytest.mark.parametrize("m,n,k,c_offset", [(1024, 1024, 4096, 0), (512, 512, 2048, 0), (300, 201, 1030, 2),
-                                            (129, 383, 2049, 6), (64, 8, 512, 0), (512, 512, 512, 2)])
+                                            (129, 383, 2049, 6), (64, 8, 2048, 0), (512, 512, 1536, 2)])
 def test_split_k_products(rt, dtype, m, n, k, c_offset):
     # Outputs that leave most compute units idle with 128 x 128 tiles and a
     # long enough reduction are split over the idle units (FP32 partials
     # added in split order): within the GEMM bar against FP64, written
     # exactly over C (guard codes around it), on 16-byte and unaligned C
-    print(f"gemm split-K dtype={dtype} {m}x{n}x{k} C offset {c_offset}", flush=True)
+    splits = gemm_plan(m, n, k, rt.compute_units)[2]
+    print(f"gemm split-K dtype={dtype} {m}x{n}x{k} C offset {c_offset}: {splits} ranges", flush=True)
+    assert splits >= 2
     a = orc.uniform(m * k, 100 + m, dtype)
     b = orc.uniform(k * n, 110 + n, dtype)
     da, db = rt.upload(a), rt.upload(b)

@@ -2,7 +2,7 @@
 allocates nothing: where xpu_gemm splits K, its FP32 partials go into a fixed
 per-GPU scratch array instead of the runtime's workspace. Called through the
 C ABI and checked bit for bit against xpu_gemm, which runs the same kernels
-with the runtime's own workspace, on two split-K calls in a row (the second
+with the runtime's own workspace, on split-K calls in a row (the later ones
 smaller, so stale partials from the first would show), plus a shape that
 needs no scratch and the size limit."""
 import ctypes
@@ -12,6 +12,7 @@ import pytest
 
 import oracle_lib as orc
 import xpu_playground_amd as xpu
+from test_gemm_plan import gemm_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -38,30 +39,25 @@ def run_both(rt, a, b, m, n, k, dtype, offset_a=0):
 
 
 def split_bytes(rt, m, n, k):
-    """The partials xpu_gemm keeps for this shape (gemm_api.cpp's rule), 0
-    when it does not split K."""
-    rows, cols = ctypes.c_uint32(), ctypes.c_uint32()
-    assert xpu.library().xpu_gemm_tile(rt.handle, m, n, ctypes.byref(rows), ctypes.byref(cols)) == 0
-    t128 = ((m + 127) // 128) * ((n + 127) // 128)
-    nslices = (k + 63) // 64
-    if (rows.value, cols.value) != (128, 128) or t128 * 2 > rt.compute_units or nslices < 8:
-        return 0
-    want = (rt.compute_units + t128 - 1) // t128
-    spl = ((nslices + want - 1) // want + 1) // 2 * 2
-    splits = (nslices + spl - 1) // spl
-    nbytes = splits * m * ((n + 3) // 4 * 4) * 4
-    return nbytes if splits >= 2 and (nslices >= 24 or nbytes <= 4 << 20) else 0
+    """The partials of the plan xpu_gemm takes for this shape (0: whole K), and
+    those of the most ranges it may take."""
+    _, _, splits, _, limit = gemm_plan(m, n, k, rt.compute_units)
+    one = m * ((n + 3) // 4 * 4) * 4
+    return (splits * one if splits >= 2 else 0), (limit * one if limit >= 2 else 0)
 
 
 def test_noalloc_matches_xpu_gemm_on_consecutive_calls(rt):
-    # first: 1024 x 1024 x 4096 bf16, 4 splits of 4 MiB (the whole array);
-    # then smaller split-K products with ragged N and K and an offset A,
-    # which reuse the array
-    cases = [(1024, 1024, 4096, xpu.BF16, 0), (300, 201, 1030, xpu.FP16, 2), (64, 40, 520, xpu.BF16, 0)]
+    # first: 1008 x 1032 x 4104 bf16, 4 ranges of nearly 4 MiB (almost the whole
+    # array); then smaller split-K products with ragged N and K and an offset
+    # A, which reuse the array
+    cases = [(1008, 1032, 4104, xpu.BF16, 0), (300, 201, 1030, xpu.FP16, 2), (512, 512, 2048, xpu.BF16, 0),
+             (129, 383, 2049, xpu.BF16, 0)]
+    before = []
     for m, n, k, dtype, off in cases:
-        need = split_bytes(rt, m, n, k)
+        need, most = split_bytes(rt, m, n, k)
         print(f"noalloc gemm {m}x{n}x{k} dtype={dtype} A offset {off}: {need} bytes of partials", flush=True)
-        assert 0 < need <= LIMIT
+        assert 0 < need <= most <= LIMIT  # K is split
+        before.append(need)
         a = orc.uniform(m * k, 31 + m, dtype)
         b = orc.uniform(k * n, 41 + n, dtype)
         ref, got = run_both(rt, a, b, m, n, k, dtype, off)
@@ -71,11 +67,12 @@ def test_noalloc_matches_xpu_gemm_on_consecutive_calls(rt):
             r = orc.decode(orc.encode(exact.astype(np.float32), dtype), dtype).astype(np.float64)
             g = orc.decode(got, dtype).astype(np.float64).reshape(m, n)
             assert np.linalg.norm(g - r) / np.linalg.norm(r) <= 1e-3
+    assert before[0] > 15 << 20 and len(set(before)) == len(before)
 
 
 def test_noalloc_without_split_needs_no_scratch(rt):
     m, n, k = 512, 512, 256  # 4 K-slices: no split
-    assert split_bytes(rt, m, n, k) == 0
+    assert split_bytes(rt, m, n, k) == (0, 0)
     a = orc.uniform(m * k, 5, xpu.BF16)
     b = orc.uniform(k * n, 6, xpu.BF16)
     ref, got = run_both(rt, a, b, m, n, k, xpu.BF16)
@@ -83,10 +80,10 @@ def test_noalloc_without_split_needs_no_scratch(rt):
 
 
 def test_noalloc_rejects_needs_above_the_array(rt):
-    # 1280 x 1280 x 2048: 100 tiles of 128 x 128, 3 splits of 6.5 MB > 16 MiB
+    # 1280 x 1280 x 2048: 100 tiles of 128 x 128, up to 3 ranges of 6.5 MB > 16 MiB
     lib = xpu.library()
     m, n, k = 1280, 1280, 2048
-    need = split_bytes(rt, m, n, k)
+    _, need = split_bytes(rt, m, n, k)
     print(f"noalloc gemm {m}x{n}x{k}: {need} bytes of partials", flush=True)
     assert need > LIMIT
     da, db, dc = rt.alloc(m * k * 2), rt.alloc(k * n * 2), rt.alloc(m * n * 2)
