@@ -1,6 +1,9 @@
 // Causal attention of a prompt chunk on the FP32 MFMA, bit for bit the decode
 // attention (attention_head in qwen3_core.hpp, qwen3/kernels.hpp:157-192), for
-// contexts of one softmax chunk (up to kAttnChunk positions).
+// contexts of one softmax chunk (up to kAttnChunk positions) and chunks that
+// start at a multiple of 16 (p0 % 16 == 0, the caller's check: a tile of 16
+// queries has to be one group of 16 positions, for the residue classes, the
+// diagonal and the last V stage).
 //
 // One block per (16 queries, head); its eight wavefronts share the LDS rows
 // of scores. v_mfma_f32_16x16x1_4b (K = 1) is one IEEE FMA per element of

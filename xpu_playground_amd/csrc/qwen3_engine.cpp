@@ -426,6 +426,7 @@ int size_prompt_buffers(xpu_qwen3 &e, bool gemm) {
 }
 
 constexpr uint32_t kBatchedChunk = 1024;
+static_assert(kBatchedChunk % 16 == 0, "xpu_q3_pf_attention_rows' query tiles start at multiples of 16");
 // LDS of xpu_q3_pf_attention_rows for contexts of up to n positions: 16 rows
 // of score codes and eight V stages (kernels/prefill_attention_rows.hip)
 uint32_t rows_attention_lds(uint32_t n) { return 16u * ((n + 63u) / 64u * 128u + 32u) + 8u * 2048u; }
@@ -685,8 +686,10 @@ int run_prefill(xpu_qwen3 &e, uint32_t P, bool head) {
                      {{8, &e.pf_q}, {8, &kc}, {8, &vc}, {8, &e.pf_a}, {4, &p0}, {4, &T}, {4, &heads}, {4, &kv},
                       {4, &max_seq}, {4, &scale}})))
           return rc;
-      } else if (e.pf_attn_rows_k && p0 + T > 128 && p0 + T <= 4096 && rows_attention_lds(p0 + T) <= rt->max_shared) {
-        // 16 queries of a head per block; contexts of one softmax chunk. Up
+      } else if (e.pf_attn_rows_k && p0 % 16 == 0 && p0 + T > 128 && p0 + T <= 4096 &&
+                 rows_attention_lds(p0 + T) <= rt->max_shared) {
+        // 16 queries of a head per block, whose first position has to be a
+        // multiple of 16; contexts of one softmax chunk. Up
         // to 128 positions its fixed cost (one 64-key tile on one wavefront,
         // ~11 us) exceeds the one-token blocks' (64 ids 11.2 against 7.8 us,
         // 128 ids 11.7 both, 256 ids 13.6 against 23.4)
