@@ -8,7 +8,7 @@ import pytest
 
 import oracle_lib as orc
 import xpu_playground_amd as xpu
-from xpu_playground_amd import Args
+from xpu_playground_amd import Args, qwen3
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +56,23 @@ def test_rows_bits(rt, epi, nc, waves, T, M, groups):
             rt.free(p)
     assert np.all(out[T * M:] == GUARD)
     assert np.array_equal(out[: T * M].reshape(T, M), want)
+
+
+def test_prompt_of_a_wide_model(rt):
+    """The K = 4096 kernels through the engine: hidden and query width 4096
+    with an intermediate size that has a kernel. Batched and stepwise prompts
+    give the same bits, below and above the token count that takes the MFMA."""
+    cfg = qwen3.preset("small")
+    cfg.hidden, cfg.intermediate, cfg.heads, cfg.kv_heads, cfg.layers, cfg.vocab = 4096, 2048, 32, 8, 1, 1000
+    eng = qwen3.Engine(cfg, max_seq=64, seed=3, gain_std=0.1, runtime=rt)
+    try:
+        for n in (20, 50):
+            ids, got = qwen3.prompt_tokens(n, 11, cfg.vocab), []
+            for form in ("stepwise", "batched"):
+                eng.set_prefill(form)
+                tokens, _, _ = eng.generate(ids, 3, stop_on_eos=False)
+                got.append((tokens, eng.logits(), eng.hidden()))
+            for a, b in zip(*got):
+                assert np.array_equal(a, b)
+    finally:
+        eng.close()

@@ -235,14 +235,19 @@ def test_command_line_matches_oracle(tmp_path):
 
 
 @pytest.mark.parametrize("preset,n_prompt,max_seq", [("small", 40, 96), ("small", 2, 16), ("small", 1, 16),
-                                                      ("small", 300, 320), ("small", 256, 272), ("small", 257, 272)])
+                                                      ("small", 300, 320), ("small", 256, 272), ("small", 257, 272),
+                                                      ("small/1", 1024, 1040), ("small/1", 1025, 1048),
+                                                      ("small/1", 1061, 1080)])
 def test_batched_prefill_bit_identical(rt, preset, n_prompt, max_seq):
-    # every prompt position in one batch per layer (chunks of 256 positions;
-    # 257 leaves the last position alone in its chunk), the last position
+    # every prompt position in one batch per layer (chunks of 1024 positions;
+    # 1025 leaves the last position alone in its chunk), the last position
     # finished by the decode step's kernels: same tokens, logits and hidden
     # state as feeding the prompt through decode one position at a time, and
-    # as the oracle, for the first generated token and after 16 more
-    cfg = orc.config(preset)
+    # as the oracle, for the first generated token and after 16 more (/1: cut
+    # to one layer, for the oracle's time)
+    cfg = orc.config(preset.split("/")[0])
+    if "/" in preset:
+        cfg.layers = int(preset.split("/")[1])
     new = min(16, max_seq - n_prompt)
     prompt = orc.tokens(n_prompt, 12, cfg.vocab)
     m = orc.Model(cfg, seed=4, gain_std=0.1, max_seq=max_seq)

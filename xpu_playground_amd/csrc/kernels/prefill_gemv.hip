@@ -189,7 +189,9 @@ XPU_DEVICE void pf_rows(const uint16_t *__restrict__ W, const uint16_t *__restri
 // spills, four wavefronts per block where eight cost registers or idle
 // blocks, eight where K = 1024 leaves room for two such blocks per compute
 // unit (128 tokens x 4096 rows: 19.9 -> 18.0 us) or K = 4096 needs the
-// weight fragments spread over more wavefronts
+// weight fragments spread over more wavefronts. K = 4096: checkpoints with
+// hidden or query width 4096 and an intermediate size of 512 {2, 4, 6, 8} (the
+// 8B shape's 12288 has no down_proj kernel, so its default prompt is stepwise)
 #define XPU_Q3_PF_ROWS(EPI, NC, HOLD, WAVES, OCC)                                                                   \
   extern "C" __global__ __launch_bounds__(64 * WAVES, OCC) void xpu_q3_pf_rows_e##EPI##_c##NC##_w##WAVES(           \
       const uint16_t *__restrict__ W, const uint16_t *__restrict__ In, uint16_t *Out, uint32_t M, uint32_t T,       \

@@ -176,7 +176,7 @@ struct xpu_qwen3 {
            *pf_h = nullptr, *pf_gu = nullptr;
   const xpu::KernelInfo *pf_silu_k = nullptr, *pf_attn_mfma_k = nullptr;
   const xpu::KernelInfo *pf_attn_rows_k = nullptr;  // 16 queries per block on the FP32 MFMA, contexts up to 4096
-  const xpu::KernelInfo *pf_attn_short_k = nullptr;  // chunks whose contexts stay within 256 positions
+  const xpu::KernelInfo *pf_attn_short_k = nullptr;  // contexts within 256 positions, where pf_attn_rows_k does not run
   const xpu::KernelInfo *pf_embed_k = nullptr, *pf_norm_k = nullptr, *pf_rope_k = nullptr, *pf_attn_k = nullptr,
                         *pf_qkv_k = nullptr, *pf_o_k = nullptr, *pf_gu_k = nullptr, *pf_down_k = nullptr;
   // rows per wavefront of those four batched GEMV kernels (their _r<R>)
