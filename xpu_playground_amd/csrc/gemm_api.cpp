@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <iomanip>
 #include <iostream>
+#include <type_traits>
 
 using xpu::set_error;
 
@@ -44,12 +45,19 @@ constexpr GemmTile kTiles[] = {{"", 256, 256, 1, 1.0, 0.0, true, true},
 // (4096^3), 224 x 256 takes outputs where it still does and cuts each unit's
 // work by 1/8 (3000 x 4097: 238 blocks instead of 204), and outputs that
 // leave most compute units idle take a smaller one.
-uint64_t tile_count(uint64_t M, uint64_t N, uint32_t rows, uint32_t cols) {
-  return ((M + rows - 1) / rows) * ((N + cols - 1) / cols);
+// (32-bit divisions: the plan is host time of every call)
+uint32_t ceil_div(uint32_t a, uint32_t b) { return a ? (a - 1) / b + 1 : 0; }
+
+uint64_t ceil_div(uint64_t a, uint32_t b) {
+  return a >> 32 ? (a + b - 1) / b : ceil_div(static_cast<uint32_t>(a), b);
+}
+
+uint64_t tile_count(uint32_t M, uint32_t N, uint32_t rows, uint32_t cols) {
+  return static_cast<uint64_t>(ceil_div(M, rows)) * ceil_div(N, cols);
 }
 
 double tile_cost(const GemmTile &t, uint32_t compute_units, uint32_t M, uint32_t n_cols) {
-  const uint64_t w = (tile_count(M, n_cols, t.rows, t.cols) + compute_units - 1) / std::max(1u, compute_units);
+  const uint64_t w = ceil_div(tile_count(M, n_cols, t.rows, t.cols), std::max(1u, compute_units));
   const double area = static_cast<double>(t.rows) * t.cols;
   return t.per_cu == 2 ? static_cast<double>(w / 2) * 2.0 * area / t.pair_rate +
                              static_cast<double>(w % 2) * area / t.solo_rate
@@ -79,8 +87,8 @@ uint32_t max_splits(uint32_t compute_units, const GemmTile &tile, uint32_t M, ui
   const uint64_t tiles = tile_count(M, N, 128, 128);
   const uint32_t slices = (K + 63) / 64;
   if (tile.rows != 128 || tile.cols != 128 || tiles * 2 > compute_units || slices < 8) return 1;
-  const uint32_t want = static_cast<uint32_t>((compute_units + tiles - 1) / tiles);
-  const uint32_t spl = ((slices + want - 1) / want + 1) / 2 * 2, splits = (slices + spl - 1) / spl;
+  const uint32_t want = ceil_div(compute_units, static_cast<uint32_t>(tiles));
+  const uint32_t spl = (ceil_div(slices, want) + 1) / 2 * 2, splits = ceil_div(slices, spl);
   const uint64_t bytes = static_cast<uint64_t>(splits) * M * ((N + 3) / 4 * 4) * 4;
   return splits >= 2 && (slices >= 24 || bytes <= (4ull << 20)) ? splits : 1;
 }
@@ -133,18 +141,20 @@ SmallPlan choose_small(uint32_t compute_units, const GemmTile &tile, uint32_t M,
   // 0.375 us is a slice's share of 128 x 128 outputs at the large tile's rate
   double best = tile_cost(tile, cus, M, N) / (128 * 128) * 0.375 * slices;
   const double mb = static_cast<double>(M) * ((N + 3) / 4 * 4) * 4e-6;
-  for (const SmallTile &t : kSmallTiles) {
+  auto consider = [&](auto index) {
+    constexpr const SmallTile &t = kSmallTiles[index];  // (its divisors are constants)
     const uint64_t tiles = tile_count(M, N, t.rows, t.cols);
     // as many ranges as fill the units, then fewer, halving
-    const uint32_t most =
-        static_cast<uint32_t>(std::min<uint64_t>(limit, std::max<uint64_t>(1, uint64_t{t.per_cu} * cus / tiles)));
+    const uint32_t most = limit == 1 || tiles >= t.per_cu * cus
+                              ? 1u
+                              : std::min(limit, t.per_cu * cus / static_cast<uint32_t>(tiles));
     for (uint32_t want = most; want >= (t.rows == 128 ? 2u : 1u); want /= 2) {
-      const uint32_t per = ((slices + want - 1) / want + t.stages - 1) / t.stages * t.stages;
-      const uint32_t splits = (slices + per - 1) / per;
-      const uint64_t w = (tiles * splits + cus - 1) / cus;
+      const uint32_t per = ceil_div(want == 1 ? slices : ceil_div(slices, want), t.stages) * t.stages;
+      const uint32_t splits = want == 1 ? 1 : ceil_div(slices, per);
+      const uint64_t w = tiles * splits <= cus ? 1 : ceil_div(tiles * splits, cus);
       double us = per * (w == 1 ? t.solo_us : static_cast<double>(w) * t.pair_us);
       if (unaligned && M <= 4 * t.rows)
-        us = std::max(us, static_cast<double>(tiles * splits) * per * (t.rows + t.cols) * 128e-6 / kUnalignedMBPerUs);
+        us = std::max(us, static_cast<double>(tiles * splits) * per * ((t.rows + t.cols) * 128e-6 / kUnalignedMBPerUs));
       if (splits >= 2) us += 1.75 + splits * (0.135 + 0.215 * mb);
       if (unaligned && !(t.rows == 128 && want == limit)) us *= kUnalignedMargin;
       if (us < best) {
@@ -152,7 +162,10 @@ SmallPlan choose_small(uint32_t compute_units, const GemmTile &tile, uint32_t M,
         plan = {&t, tiles, splits, per};
       }
     }
-  }
+  };
+  consider(std::integral_constant<size_t, 0>{});
+  consider(std::integral_constant<size_t, 1>{});
+  consider(std::integral_constant<size_t, 2>{});
   return plan;
 }
 
