@@ -30,8 +30,9 @@
 // 3072; measured at 2048 tokens 38 and 42, against 20-23 for pf_gemv. Each
 // pair of slots unpacks all its operands, then issues its MFMAs back to back,
 // then folds: alternating one MFMA with its two unpacks cost 6%.
-// At 128 tokens (us, 0.6B rows): QKV 29.0 -> 20.2, o_proj 16.9 -> 13.8,
-// [gate; up] 47.5 -> 32.7, down 25.3 -> 17.8.
+// At 128 tokens (us, 0.6B rows): QKV 29.0 -> 20.3, o_proj 16.9 -> 13.7,
+// [gate; up] 47.5 -> 33.8, down 25.3 -> 19.3. That rate allows 12, 5, 18 and 7
+// there: a block's few token tiles do not cover its first weight loads.
 #include "qwen3_core.hpp"
 
 namespace {

@@ -935,7 +935,7 @@ extern "C" __global__ __launch_bounds__(256) void xpu_q3_attn_scores(
 // trace: 7.9 us a launch against 8.1 with V first). Cycles of a wavefront
 // (median, 0.6B, 2048 positions, stamps build): 21.7K (9.4 us a launch) with V
 // tiles through LDS and the denominator on one wavefront, 18.8K (8.2 us) with
-// 2-byte loads of one dim per thread, 12.2K here (7.0 us).
+// 2-byte loads of one dim per thread, 11.4K here (6.8 us).
 extern "C" __global__ __launch_bounds__(256, 1) void xpu_q3_attn_pv(
     const float *__restrict__ scores, const float *__restrict__ maxima, const uint16_t *__restrict__ vcache,
     uint16_t *__restrict__ out, const uint32_t *__restrict__ state, uint32_t heads, uint32_t kv_heads,
