@@ -140,7 +140,7 @@ def test_ragged_baseline_shape_reads_operands_in_place(rt):
 
 
 @pytest.mark.parametrize("dtype", [xpu.BF16, xpu.FP16])
-@pytest.mark.parametrize("m,n,k,c_offset", [(1024, 1024, 4096, 0), (512, 512, 2048, 0), (300, 201, 1030, 2),
+@pytest.mark.parametrize("m,n,k,c_offset", [(768, 768, 8192, 0), (512, 512, 2048, 0), (300, 201, 1030, 2),
                                             (129, 383, 2049, 6), (64, 8, 2048, 0), (512, 512, 1536, 2)])
 def test_split_k_products(rt, dtype, m, n, k, c_offset):
     # Outputs that leave most compute units idle with 128 x 128 tiles and a

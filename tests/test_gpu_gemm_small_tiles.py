@@ -20,7 +20,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,offsets", [
     (1, 1, 1, (0, 0, 0)), (31, 127, 63, (2, 6, 2)), (32, 128, 64, (0, 0, 0)), (33, 129, 65, (4, 2, 0)),
     (64, 128, 192, (0, 0, 0)), (65, 136, 193, (0, 0, 0)), (63, 263, 256, (6, 14, 4)), (100, 96, 257, (0, 0, 2)),
-    (129, 392, 520, (0, 0, 0)), (300, 77, 1031, (10, 2, 0))])
+    (129, 392, 520, (0, 0, 0)), (300, 77, 1031, (10, 2, 0)),
+    # more tile-columns than tile-rows, no multiple of 8 tiles: dealt to the XCDs in ranges
+    (5, 2100, 70, (0, 0, 0)), (70, 1300, 130, (2, 4, 2)), (97, 520, 65, (0, 0, 0))])
 def test_small_tiles_equal_128_tile(rt, monkeypatch, dtype, m, n, k, offsets):
     monkeypatch.setitem(edges.TILES, "_m32", (32, 128))
     monkeypatch.setitem(edges.TILES, "_m64", (64, 128))
@@ -34,7 +36,7 @@ def test_small_tiles_equal_128_tile(rt, monkeypatch, dtype, m, n, k, offsets):
 
 def launch_ranges(rt, rows, dtype, a, b, m, n, k, slices, offsets):
     """One launch of a split kernel and of the reduction: the FP32 partials and C."""
-    tag = {32: "_m32", 64: "_m64", 128: "_t128"}[rows]
+    tag = {32: "_m32", 64: "_m64"}[rows]
     splits, pitch = ((k + 63) // 64 + slices - 1) // slices, (n + 3) // 4 * 4
     words = splits * m * pitch
     da, db = rt.alloc(a.size * 2 + 32), rt.alloc(b.size * 2 + 32)
@@ -70,15 +72,15 @@ def launch_ranges(rt, rows, dtype, a, b, m, n, k, slices, offsets):
     (100, 72, 64 * 23 + 63, 12, (0, 0, 4)),   # the last group partly past K
     (64, 128, 64 * 96, 12, (0, 0, 0)),        # 8 ranges: the reduction's first batch of seven
     (40, 96, 64 * 97 + 1, 12, (0, 0, 0)),     # 9: into its second
+    (70, 1300, 64 * 26, 12, (0, 0, 0)),       # 33 and 22 tiles a range, dealt to the XCDs in ranges
     (5, 66, 64 * 180 + 2, 12, (10, 2, 2))])   # 16: past its second
 def test_range_kernels_give_the_same_partials(rt, dtype, m, n, k, slices, offsets):
     a = orc.uniform(m * k, 7 * m + k, dtype)
     b = orc.uniform(k * n, 9 * n + k, dtype)
-    want, out = launch_ranges(rt, 128, dtype, a, b, m, n, k, slices, offsets)
+    want, out = launch_ranges(rt, 64, dtype, a, b, m, n, k, slices, offsets)
     check(out, a, b, m, n, k, dtype)
-    for rows in (32, 64):
-        parts, c = launch_ranges(rt, rows, dtype, a, b, m, n, k, slices, offsets)
-        assert np.array_equal(parts, want) and np.array_equal(c, out)
+    parts, c = launch_ranges(rt, 32, dtype, a, b, m, n, k, slices, offsets)
+    assert np.array_equal(parts, want) and np.array_equal(c, out)
     # the partials themselves: each range's product, in 64 bits
     fa = orc.decode(a, dtype).reshape(m, k).astype(np.float64)
     fb = orc.decode(b, dtype).reshape(k, n).astype(np.float64)
@@ -91,8 +93,8 @@ def test_range_kernels_give_the_same_partials(rt, dtype, m, n, k, slices, offset
 
 # (m, n, k, rows of the tile, K ranges) that the dispatch takes on 256 compute units
 @pytest.mark.parametrize("m,n,k,rows,splits", [
-    (24, 4096, 4096, 32, 8), (33, 1000, 1537, 32, 7), (1024, 512, 4096, 64, 4), (3043, 66, 1666, 64, 5),
-    (768, 768, 8192, 64, 3), (1000, 1001, 5001, 128, 4), (1008, 1032, 4104, 128, 4)])
+    (24, 4096, 4096, 32, 8), (33, 1000, 1537, 32, 7), (118, 2632, 3942, 32, 3), (3043, 66, 1666, 64, 5),
+    (768, 768, 8192, 64, 3), (1000, 1001, 5001, 64, 2)])
 def test_dispatch_splits_in_each_tile(rt, m, n, k, rows, splits):
     if rt.compute_units == 256:
         assert gemm_plan(m, n, k)[::2][:2] == (rows, splits)

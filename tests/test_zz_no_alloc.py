@@ -47,10 +47,10 @@ def split_bytes(rt, m, n, k):
 
 
 def test_noalloc_matches_xpu_gemm_on_consecutive_calls(rt):
-    # first: 1008 x 1032 x 4104 bf16, 4 ranges of nearly 4 MiB (almost the whole
-    # array); then smaller split-K products with ragged N and K and an offset
-    # A, which reuse the array
-    cases = [(1008, 1032, 4104, xpu.BF16, 0), (300, 201, 1030, xpu.FP16, 2), (512, 512, 2048, xpu.BF16, 0),
+    # first: 1088 x 636 x 6427 bf16, 3 ranges of 2.6 MiB (no plan of a shape that
+    # is accepted takes much more); then smaller split-K products with ragged N
+    # and K and an offset A, which reuse the array
+    cases = [(1088, 636, 6427, xpu.BF16, 0), (300, 201, 1030, xpu.FP16, 2), (512, 512, 2048, xpu.BF16, 0),
              (129, 383, 2049, xpu.BF16, 0)]
     before = []
     for m, n, k, dtype, off in cases:
@@ -67,7 +67,7 @@ def test_noalloc_matches_xpu_gemm_on_consecutive_calls(rt):
             r = orc.decode(orc.encode(exact.astype(np.float32), dtype), dtype).astype(np.float64)
             g = orc.decode(got, dtype).astype(np.float64).reshape(m, n)
             assert np.linalg.norm(g - r) / np.linalg.norm(r) <= 1e-3
-    assert before[0] > 15 << 20 and len(set(before)) == len(before)
+    assert before[0] > 7 << 20 and len(set(before)) == len(before)
 
 
 def test_noalloc_without_split_needs_no_scratch(rt):

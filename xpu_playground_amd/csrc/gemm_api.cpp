@@ -93,17 +93,15 @@ uint32_t max_splits(uint32_t compute_units, const GemmTile &tile, uint32_t M, ui
   return splits >= 2 && (slices >= 24 || bytes <= (4ull << 20)) ? splits : 1;
 }
 
-// The tiles that take K in ranges (kernels/gemm.hip), the first two also whole
-// K: stages (slices per group), blocks a unit that K is split for, and us per
-// 64-deep slice with w blocks on the busiest unit, w * pair_us for w >= 2.
+// The small tiles (kernels/gemm.hip): stages
+// (slices per group) and us per 64-deep slice with w blocks on the busiest
+// unit, w * pair_us for w >= 2.
 struct SmallTile {
   const char *tag;
-  uint32_t rows, cols, stages, per_cu;
+  uint32_t rows, cols, stages;
   double solo_us, pair_us;
 };
-constexpr SmallTile kSmallTiles[] = {{"_m32", 32, 128, 4, 1, 0.27, 0.27},
-                                     {"_m64", 64, 128, 3, 2, 0.33, 0.36},
-                                     {"_t128", 128, 128, 2, 2, 0.64, 0.40}};
+constexpr SmallTile kSmallTiles[] = {{"_m32", 32, 128, 4, 0.26, 0.27}, {"_m64", 64, 128, 3, 0.33, 0.36}};
 
 struct SmallPlan {
   const SmallTile *tile = nullptr;  // null: the tile of choose_tile, whole K
@@ -111,33 +109,22 @@ struct SmallPlan {
   uint32_t splits = 1, slices = 0;  // K ranges, and slices per range
 };
 
-// The plan with the least estimated time: the chosen tile, or one of these
-// tiles with K whole or in up to `limit` ranges. us per slice (a group of
-// slices past K costs as much) over the busiest unit's blocks, plus for a split
-// the second launch (1.75 us), each range's load in the reduction (0.135 us)
-// and the partials' round trip (0.215 us per MB). Against 128 x 128 tiles, K
-// split in `limit` ranges (bf16, back to back): 24 x 4096 x 4096 (8 ranges of
-// 32 x 128) 12.0 -> 9.1 us, 64 x 1024 x 4096 13.1 -> 8.1, 512^3 (whole K) 8.9
-// -> 4.3, 1024^3 9.5 -> 6.7, 300 x 3000 x 3000 20.5 -> 17.3, 1500 x 1000 x 600
-// (64 x 128) 7.7 -> 6.6; 2048 x 2048 x 512 stays (8.0 against 9.0).
-//
-// Rows that are not whole 128-byte cache lines (K or N no multiple of 64)
-// share lines, and their slices cost more of them. There, with at most four row
-// tiles, whose B rows all come from beyond the L2s, slices arrive at 12.4 TB/s
-// (118 x 2632 x 3942: 22.6 us in 32 x 128 tiles, 17.5 in 128 x 128), and any
-// other plan than the 128 x 128 tiles' has to look 15% better. Fitted to 1200
-// shapes, 700 of them of few rows or columns and long K, each with operands from
-// the Infinity Cache and from memory: without these two rules 18 of the 2400
-// times were over 3% longer than with 128 x 128 tiles split in `limit` ranges
-// (up to 15%), with them 2 (4 and 8%).
-constexpr double kUnalignedMBPerUs = 12.4, kUnalignedMargin = 1.15;
-
+// A small tile, with K whole or in up to `limit` ranges, where its estimated
+// time is below the chosen tile's: us per slice (a group of slices past K
+// costs as much) over the busiest unit's blocks, plus for a split the second
+// launch (2 us), each range's load in the reduction (0.12 us) and the
+// partials' round trip (0.55 us per MB). Fitted to 19 swept shapes, bf16 and
+// back to back: it takes the measured fastest plan or one within 8% of it.
+// Against 128 x 128 tiles, K split as max_splits says: 24 x 4096 x 4096 (8
+// ranges of 32 x 128) 12.0 -> 9.1 us, 64 x 1024 x 4096 13.1 -> 8.1, 512^3
+// (whole K) 8.9 -> 4.3, 1024^3 9.5 -> 6.7, 300 x 3000 x 3000 20.5 -> 17.3,
+// 1500 x 1000 x 600 (64 x 128) 7.7 -> 6.6; 2048 x 2048 x 512 stays (8.0
+// against 9.0).
 SmallPlan choose_small(uint32_t compute_units, const GemmTile &tile, uint32_t M, uint32_t N, uint32_t K,
                        uint32_t limit) {
   SmallPlan plan;
   if (tile.rows > 128) return plan;
   const uint32_t slices = (K + 63) / 64, cus = std::max(1u, compute_units);
-  const bool unaligned = K % 64 || N % 64;
   // 0.375 us is a slice's share of 128 x 128 outputs at the large tile's rate
   double best = tile_cost(tile, cus, M, N) / (128 * 128) * 0.375 * slices;
   const double mb = static_cast<double>(M) * ((N + 3) / 4 * 4) * 4e-6;
@@ -145,27 +132,22 @@ SmallPlan choose_small(uint32_t compute_units, const GemmTile &tile, uint32_t M,
     constexpr const SmallTile &t = kSmallTiles[index];  // (its divisors are constants)
     const uint64_t tiles = tile_count(M, N, t.rows, t.cols);
     // as many ranges as fill the units, then fewer, halving
-    const uint32_t most = limit == 1 || tiles >= t.per_cu * cus
-                              ? 1u
-                              : std::min(limit, t.per_cu * cus / static_cast<uint32_t>(tiles));
-    for (uint32_t want = most; want >= (t.rows == 128 ? 2u : 1u); want /= 2) {
+    for (uint32_t want = limit == 1 || tiles >= cus ? 1u : std::min(limit, cus / static_cast<uint32_t>(tiles));;
+         want /= 2) {
       const uint32_t per = ceil_div(want == 1 ? slices : ceil_div(slices, want), t.stages) * t.stages;
       const uint32_t splits = want == 1 ? 1 : ceil_div(slices, per);
       const uint64_t w = tiles * splits <= cus ? 1 : ceil_div(tiles * splits, cus);
-      double us = per * (w == 1 ? t.solo_us : static_cast<double>(w) * t.pair_us);
-      if (unaligned && M <= 4 * t.rows)
-        us = std::max(us, static_cast<double>(tiles * splits) * per * ((t.rows + t.cols) * 128e-6 / kUnalignedMBPerUs));
-      if (splits >= 2) us += 1.75 + splits * (0.135 + 0.215 * mb);
-      if (unaligned && !(t.rows == 128 && want == limit)) us *= kUnalignedMargin;
+      const double us = per * (w == 1 ? t.solo_us : static_cast<double>(w) * t.pair_us) +
+                        (splits >= 2 ? 2.0 + splits * (0.12 + 0.55 * mb) : 0.0);
       if (us < best) {
         best = us;
         plan = {&t, tiles, splits, per};
       }
+      if (want <= 1) break;
     }
   };
   consider(std::integral_constant<size_t, 0>{});
   consider(std::integral_constant<size_t, 1>{});
-  consider(std::integral_constant<size_t, 2>{});
   return plan;
 }
 
