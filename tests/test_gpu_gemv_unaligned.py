@@ -52,5 +52,5 @@ def test_aligned_rows_with_and_without_ends(rt, dtype, m, k):
 
 
 def test_many_rows_of_whole_batches(rt):
-    """More than 64 rows a compute unit: one block a unit instead of four."""
-    test_unaligned_rows(rt, xpu.BF16, 64 * rt.compute_units + 3, 5120, 0, 0)
+    """A matrix past 400 MB: one block a compute unit instead of four."""
+    test_unaligned_rows(rt, xpu.BF16, (200 << 20) // 7168 + 1, 7168, 0, 0)

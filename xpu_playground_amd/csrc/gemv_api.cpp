@@ -47,13 +47,14 @@ int plan_gemv(const xpu_runtime &rt, int dtype, const void *A, const void *x, ui
   // with two to four, 32768 x 8192 79.4 against 79.3-81.1): its pipeline keeps
   // the loads in flight. Up to four, as the LDS allows, where it drains at every
   // row's end instead: 151936 x 1024 86.5 -> 52.8 us, 20000 x 1024 12.7 -> 8.4,
-  // 16384 x 500 10.0 -> 5.2, 12000 x 10000 58.5 -> 38.9; and for up to 64 rows a
-  // unit of K = 5120 or 7168 (16384 rows 27.4 -> 26.4 and 36.2 -> 36.0; 65536
-  // rows 95.0 against 96.9 and 129.5 against 134.5 with one and four).
+  // 16384 x 500 10.0 -> 5.2, 12000 x 10000 58.5 -> 38.9; and for K = 5120 or
+  // 7168 up to 400 MB, well past the Infinity Cache (16384 rows 27.4 -> 26.4 and
+  // 36.2 -> 36.0, 40000 x 5120 62.3 -> 61.2; with one and four blocks 32768 x
+  // 7168 67.5 against 69.1, 65536 rows 95.0 against 96.9 and 129.5 against 134.5).
   const uint64_t tiles = (static_cast<uint64_t>(M) + 4 * rows - 1) / (4 * rows);
   const bool whole = K >= 4096 && K % (short_rows ? 1024 : 2048) == 0;
   const uint32_t per_cu =
-      whole && (K % 2048 == 0 || M > 64 * rt.compute_units)
+      whole && (K % 2048 == 0 || static_cast<uint64_t>(M) * K > 200u << 20)
           ? 1u
           : plan.shared ? std::min(4u, std::max(1u, rt.max_shared / plan.shared)) : 1u;
   plan.grid = static_cast<uint32_t>(std::min<uint64_t>(tiles, uint64_t{rt.compute_units} * per_cu));
