@@ -132,8 +132,9 @@ XPU_DEVICE void gemv_load_batch(u32x4 (&buf)[U][R], const uint16_t *const (&rows
 // caller with gemv_load_batch so that its latency overlaps other work; it is
 // only used when K has at least U full chunks. EARLY: the chunk that crosses K
 // and, for U = 2, the full chunk left over after the batches are loaded ahead
-// of them, so that a row does not wait for its end on its own.
-template <int DT, int R, int U, bool VEC, bool PAIRED = false, bool EARLY = false>
+// of them, so that a row does not wait for its end on its own. CACHED: a row's
+// first batch with cached loads instead of streaming ones.
+template <int DT, int R, int U, bool VEC, bool PAIRED = false, bool EARLY = false, bool CACHED = false>
 XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, uint32_t K,
                                 uint32_t M, const uint16_t *xs, uint32_t row0, float (&out)[R],
                                 uint32_t pair_offset, const u32x4 (&first)[U][R], bool use_first) {
@@ -181,9 +182,7 @@ XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, ui
 #pragma unroll
         for (int r = 0; r < R; ++r) b0[u][r] = first[u][r];
     } else {
-      // cached where a row's end is loaded ahead: bf16 40000 x 4608 54.9 us
-      // against 56.5 with streaming loads, 16384 x 2048 11.9 against 12.1
-      gemv_load_batch<R, U, VEC, !EARLY>(b0, rows, 0);
+      gemv_load_batch<R, U, VEC, !CACHED>(b0, rows, 0);
     }
     while (true) {
       if (j + 2 * U > nfull) { fma_batch(b0, j); j += U; break; }
@@ -237,11 +236,11 @@ XPU_DEVICE void gemv_rows_first(const uint16_t *__restrict__ A, uint64_t lda, ui
   for (int r = 0; r < R; ++r) out[r] = wave_butterfly(fold8(acc[r]));
 }
 
-template <int DT, int R, int U, bool VEC, bool EARLY = false>
+template <int DT, int R, int U, bool VEC, bool EARLY = false, bool CACHED = false>
 XPU_DEVICE void gemv_rows(const uint16_t *__restrict__ A, uint64_t lda, uint32_t K, uint32_t M,
                           const uint16_t *xs, uint32_t row0, float (&out)[R]) {
   u32x4 unused[U][R];
-  gemv_rows_first<DT, R, U, VEC, false, EARLY>(A, lda, K, M, xs, row0, out, 0, unused, false);
+  gemv_rows_first<DT, R, U, VEC, false, EARLY, CACHED>(A, lda, K, M, xs, row0, out, 0, unused, false);
 }
 
 }  // namespace xpu
